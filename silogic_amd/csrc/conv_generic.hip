@@ -439,6 +439,10 @@ int conv_generic_params(int node, int depth, int arity) {
   return nn * ((node == SLG_NODE_GATE16 || node == SLG_NODE_WALSH) ? 4 : (1 << A));
 }
 
+int conv_generic_leaves(int node, int depth, int arity) {
+  return ipow((node == SLG_NODE_GATE16 || node == SLG_NODE_WALSH) ? 2 : arity, depth);
+}
+
 int conv_generic_fwd(const float* x, int64_t B, int64_t C, int64_t H, int64_t W, int64_t N,
                      int node, int depth, int arity, int K, int kernel, int pad, bool pool,
                      const float* np, const float* w, const int* cm, const int* ch, const int* cw,

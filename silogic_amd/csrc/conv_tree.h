@@ -104,6 +104,7 @@ __device__ inline float conv_tree_eval(const float (&v)[NLEAF], const float* par
 // coefficients times 1/tau) or 2^arity (LUT values).
 bool conv_generic_supported(int node, int depth, int arity);
 int conv_generic_params(int node, int depth, int arity);
+int conv_generic_leaves(int node, int depth, int arity);
 int conv_generic_fwd(const float* x, int64_t B, int64_t C, int64_t H, int64_t W, int64_t N,
                      int node, int depth, int arity, int K, int kernel, int pad, bool pool,
                      const float* np, const float* w, const int* cm, const int* ch, const int* cw,
