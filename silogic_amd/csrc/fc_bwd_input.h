@@ -4,7 +4,7 @@
 // side*OUT + o), the candidates cand [OUT,nsides,K] and weights w,
 //   gx[b][i] = sum over references (o, side, k) with cand = i of
 //              w[o,side,k] * gbr[b][side*OUT + o],
-// summed in ascending reference order (the same bits on every call).
+// summed in a fixed order (the same bits on every call).
 #pragma once
 
 #include "slg_common.h"

@@ -1,0 +1,408 @@
+// Input gradient of the FC soft layers (fc_bwd_input.h): the transposed
+// problem of the forward, in the forward's form. The operand gradients of a
+// tile of 4 samples sit in LDS (16 bytes a row, the rows of one pass at a
+// time) and every input gathers its references from there: 16-byte reads at
+// random rows, 76 bytes a clock and CU measured, where gathering sample-minor
+// rows through L2 ran at 12 (they pass its 4 MB per XCD) and needed a
+// transpose of all operand gradients before. Measured at 10000 -> 10000,
+// K = 8, B = 4096: transpose and gather 474 us -> 217 us (4 tiles a CU, each
+// two passes of staging 160 KB at the memory's rate, about 8 us, and of
+// gathering from it at the LDS rate, about 8 us, with the whole LDS in use
+// nothing of the next pass to overlap with); 4000 -> 4000 LUT4, B = 1024: 88
+// -> 45 us. 512 threads of 256 registers: with 1024 of 128 the entry stream
+// spilled (255-303 us).
+//
+// Inputs are grouped by block (the workgroup's share of the inputs) and pass
+// (the rows in LDS together). Within a group they are ordered by reference
+// count, so the 64 lanes of a wave have equally long lists; a chunk of 64
+// inputs stores its lists side by side ([step][lane], one coalesced 512-byte
+// load a step) and a wave's chunks follow each other, so that its entries are
+// one stream, loaded 12 steps ahead (a chunk is about 10 steps: started
+// chunk by chunk, its first loads' latency was half of the gather). An input's sum stays with a lane through a pass; between
+// passes, and before the rows are written, the sums change places through
+// LDS. Inputs of more than kHeavy references (narrow inputs under wide
+// layers) take a wave each instead.
+//
+// Every sum has a fixed order: passes ascending, references ascending in a
+// pass (heavy inputs: lane by lane, then over the lanes).
+#include "fc_bwd_input.h"
+#include "fc_soft_common.h"
+#include "ref_table.h"
+
+namespace slg {
+
+constexpr int kIgThreads = 512;
+constexpr int kIgSlots = 20;                             // inputs per thread
+constexpr int kIgBlock = kIgThreads * kIgSlots;          // inputs per block, at most
+constexpr int kIgRows = 10236;                           // rows per pass, at most: with a zero
+                                                         // row 16 B each in 160 KB of LDS
+constexpr int kIgWaves = kIgThreads / 64;
+constexpr int kIgStep = 4;                               // entries a lane takes at a time
+constexpr int kHeavy = 512;                              // references of a lane's list, at most
+
+struct IgArgs {
+  int B, IN, R2, OUT, NS, K;
+  int NB, IB;      // input blocks, inputs per block
+  int NP, RB;      // passes, rows per pass
+  int64_t R;
+};
+
+// Steps of a chunk whose longest list has n entries: whole blocks of kIgStep.
+__device__ inline int ig_steps(int n) { return (n + kIgStep - 1) / kIgStep * kIgStep; }
+// A group's entries past its references: its longest list in the first
+// chunk (lists descend, so each other chunk's padding is at most the
+// references of the chunk before it) and the rounding of every chunk.
+__host__ __device__ inline int ig_slack(int IB) {
+  return 64 * kHeavy + 64 * kIgStep * ((IB + 63) / 64);
+}
+
+// group = pass * NB + block; key = group * IB + input within the block
+__global__ void __launch_bounds__(256) ig_keys_kernel(IgArgs a, const int* __restrict__ cand,
+                                                      int* __restrict__ keys) {
+  const int r = blockIdx.x * 256 + threadIdx.x;
+  if (r >= a.R) return;
+  const int i = min(max(cand[r], 0), a.IN - 1);
+  const int SK = a.NS * a.K, o = r / SK, side = (r - o * SK) / a.K;
+  const int q = i / a.IB;
+  keys[r] = ((side * a.OUT + o) / a.RB * a.NB + q) * a.IB + (i - q * a.IB);
+}
+
+// One workgroup per group: its inputs in descending order of their counts
+// (by a counting sort; the place among equal counts does not matter to any
+// sum). perm [group][IB]: each slot's input | its count << 16, and the heavy
+// inputs from the end; slot [key] (heavy inputs: -1); off: the first entry of
+// each chunk of 64 slots.
+__global__ void __launch_bounds__(1024) ig_slots_kernel(IgArgs a, const int* __restrict__ start,
+                                                        int* __restrict__ perm,
+                                                        int* __restrict__ slot,
+                                                        int* __restrict__ off,
+                                                        int* __restrict__ heavy) {
+  __shared__ int hist[kHeavy + 2], at[kHeavy + 2], part[16];
+  const int g = blockIdx.x, q = g % a.NB;
+  const int n = min(a.IB, a.IN - q * a.IB);  // inputs of the block
+  const int t = threadIdx.x;
+  const int* s = start + (int64_t)g * a.IB;
+  int* pm = perm + (int64_t)g * a.IB;
+  int* sl = slot + (int64_t)g * a.IB;
+  for (int i = t; i < kHeavy + 2; i += 1024) hist[i] = 0;
+  __syncthreads();
+  for (int i = t; i < n; i += 1024) atomicAdd(&hist[min(s[i + 1] - s[i], kHeavy + 1)], 1);
+  __syncthreads();
+  if (t < 64) {  // at[c] = inputs of more than c references, heavy ones aside
+    int run = 0;
+    for (int hi = kHeavy; hi >= 0; hi -= 64) {
+      const int c = hi - t;
+      const int v = c >= 0 ? hist[c] : 0;
+      int x = v;
+#pragma unroll
+      for (int d = 1; d < 64; d <<= 1) {
+        const int y = __shfl_up(x, d, 64);
+        if (t >= d) x += y;
+      }
+      if (c >= 0) at[c] = run + x - v;
+      run += __shfl(x, 63, 64);
+    }
+    if (t == 0) {
+      heavy[g] = hist[kHeavy + 1];
+      at[kHeavy + 1] = a.IB - hist[kHeavy + 1];
+    }
+  }
+  __syncthreads();
+  for (int i = t; i < n; i += 1024) {
+    const int c = s[i + 1] - s[i];
+    const int p = atomicAdd(&at[min(c, kHeavy + 1)], 1);
+    pm[p] = c > kHeavy ? i : i | (c << 16);
+    sl[i] = c > kHeavy ? -1 : p;
+  }
+  __threadfence_block();
+  __syncthreads();
+  // chunk offsets: a chunk is as long as its first slot's list, in whole
+  // blocks; chunk w + kIgWaves j is the j-th of wave w, wave by wave
+  const int m = n - hist[kHeavy + 1], nc = (m + 63) >> 6, NC = (a.IB + 63) >> 6;
+  const int c = t / kIgSlots + kIgWaves * (t % kIgSlots);
+  const int len = t < kIgWaves * kIgSlots && c < nc ? 64 * ig_steps(pm[64 * c] >> 16) : 0;
+  int x = len;
+  const int lane = t & 63, wave = t >> 6;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int y = __shfl_up(x, d, 64);
+    if (lane >= d) x += y;
+  }
+  if (lane == 63) part[wave] = x;
+  __syncthreads();
+  int base = s[0] + g * ig_slack(a.IB);
+  for (int w = 0; w < wave; ++w) base += part[w];
+  if (t < kIgWaves * kIgSlots && c < NC) off[(int64_t)g * NC + c] = base + x - len;
+}
+
+// Entries (LDS byte offset of the row within its pass, weight) of each
+// reference: a chunk's lists [step][lane], heavy inputs' lists as they lie.
+__global__ void __launch_bounds__(256) ig_entries_kernel(IgArgs a, const int* __restrict__ sorted,
+                                                         const int* __restrict__ keys,
+                                                         const int* __restrict__ start,
+                                                         const int* __restrict__ slot,
+                                                         const int* __restrict__ off,
+                                                         const float* __restrict__ w,
+                                                         int2* __restrict__ ent,
+                                                         int2* __restrict__ ent_heavy) {
+  const int j = blockIdx.x * 256 + threadIdx.x;
+  if (j >= a.R) return;
+  const int r = sorted[j], key = keys[r];
+  const int SK = a.NS * a.K, o = r / SK, side = (r - o * SK) / a.K;
+  const int row = side * a.OUT + o;
+  const int2 e = make_int2((row - row / a.RB * a.RB) * 16, __float_as_int(w[r]));
+  const int s = slot[key];
+  if (s < 0) {
+    ent_heavy[j] = e;
+  } else {
+    const int NC = (a.IB + 63) >> 6;
+    const int64_t at = off[(int64_t)(key / a.IB) * NC + (s >> 6)] + (int64_t)(j - start[key]) * 64 + (s & 63);
+    ent[at] = e;
+  }
+}
+
+__global__ void __launch_bounds__(kIgThreads)
+ig_gather_kernel(IgArgs a, const float* __restrict__ gbr, const int* __restrict__ start,
+                 const int* __restrict__ perm, const int* __restrict__ off,
+                 const int* __restrict__ heavy, const int2* __restrict__ ent,
+                 const int2* __restrict__ ent_heavy, float* __restrict__ gx) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  f32x4* rows = reinterpret_cast<f32x4*>(smem);
+  const int q = (int)(blockIdx.x % (unsigned)a.NB), tile = (int)(blockIdx.x / (unsigned)a.NB);
+  const int b0 = tile * 4, nb = min(4, a.B - b0);
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int i0 = q * a.IB, n = min(a.IB, a.IN - i0);
+  const int NC = (a.IB + 63) >> 6;
+  f32x4 acc[kIgSlots];
+#pragma unroll
+  for (int j = 0; j < kIgSlots; ++j) acc[j] = (f32x4)0.0f;
+  for (int p = 0; p < a.NP; ++p) {
+    const int g = p * a.NB + q;
+    const int* s = start + (int64_t)g * a.IB;
+    const int* pm = perm + (int64_t)g * a.IB;
+    const int nh = heavy[g], m = n - nh;
+    // this thread's slots (input | count << 16; past the group: count 0) and
+    // the first blocks of the wave's entries
+    int pv[kIgSlots];
+#pragma unroll
+    for (int j = 0; j < kIgSlots; ++j) {
+      const int k = (wave + kIgWaves * j) * 64 + lane;
+      pv[j] = k < m ? pm[k] : -1;
+    }
+    const int2* e = ent + __builtin_amdgcn_readfirstlane(wave < NC ? off[(int64_t)g * NC + wave] : 0);
+    int2 e0[kIgStep], e1[kIgStep], e2[kIgStep];
+#pragma unroll
+    for (int u = 0; u < kIgStep; ++u) {
+      e0[u] = e[u * 64 + lane];
+      e1[u] = e[(kIgStep + u) * 64 + lane];
+      e2[u] = e[(2 * kIgStep + u) * 64 + lane];
+    }
+    if (p) {  // the sums so far, from their inputs' places to this pass's slots
+#pragma unroll
+      for (int j = 0; j < kIgSlots; ++j)
+        if (pv[j] >= 0) acc[j] = rows[pv[j] & 0xffff];
+      for (int h = wave; h < nh; h += kIgWaves) {
+        const int i = pm[a.IB - nh + h];
+        if (lane < nb)
+          gx[(int64_t)(b0 + lane) * a.IN + i0 + i] = reinterpret_cast<const float*>(rows + i)[lane];
+      }
+      __syncthreads();
+    }
+    // stage rows [p RB, p RB + nr) of the tile's samples, then a zero row
+    const int c0 = p * a.RB, nr = min(a.RB, a.R2 - c0);
+    const float* src = gbr + (int64_t)b0 * a.R2 + c0;
+    if (((a.R2 | c0 | nr) & 3) == 0) {
+      constexpr int NL = 3;  // 16-byte loads of a row in flight per thread, times 4 samples
+      for (int k0 = tid; k0 < nr >> 2; k0 += NL * kIgThreads) {
+        float4 t[NL][4];
+#pragma unroll
+        for (int l = 0; l < NL; ++l) {
+          const int k = k0 + l * kIgThreads;
+#pragma unroll
+          for (int v = 0; v < 4; ++v)
+            t[l][v] = v < nb && k < nr >> 2 ? ld_stream4(src + (int64_t)v * a.R2 + 4 * k)
+                                            : make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+#pragma unroll
+        for (int l = 0; l < NL; ++l) {
+          const int k = k0 + l * kIgThreads;
+          if (k < nr >> 2) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+              rows[4 * k + u] = f32x4{lanev(t[l][0], u), lanev(t[l][1], u), lanev(t[l][2], u),
+                                      lanev(t[l][3], u)};
+          }
+        }
+      }
+    } else {
+      for (int k = tid; k < nr; k += kIgThreads) {
+        f32x4 t;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) t[v] = v < nb ? src[(int64_t)v * a.R2 + k] : 0.0f;
+        rows[k] = t;
+      }
+    }
+    if (tid == 0) rows[nr] = (f32x4)0.0f;
+    __syncthreads();
+    auto row = [&](int byte) { return *reinterpret_cast<const f32x4*>(smem + byte); };
+#pragma unroll
+    for (int j = 0; j < kIgSlots; ++j) {
+      const int cnt = pv[j] >= 0 ? pv[j] >> 16 : 0;
+      const int L = ig_steps(__builtin_amdgcn_readfirstlane(cnt));
+      const int least = __builtin_amdgcn_readlane(cnt, 63);
+      f32x4 sum = acc[j];
+      for (int t0 = 0; t0 < L; t0 += kIgStep) {
+        int2 cur[kIgStep];
+#pragma unroll
+        for (int u = 0; u < kIgStep; ++u) cur[u] = e0[u];
+        e += kIgStep * 64;
+#pragma unroll
+        for (int u = 0; u < kIgStep; ++u) {
+          e0[u] = e1[u];
+          e1[u] = e2[u];
+          e2[u] = e[(2 * kIgStep + u) * 64 + lane];
+        }
+        if (t0 + kIgStep > least) {  // past some lanes' lists: the zero row
+#pragma unroll
+          for (int u = 0; u < kIgStep; ++u)
+            if (t0 + u >= cnt) cur[u] = make_int2(nr * 16, 0);
+        }
+        f32x4 v[kIgStep];
+#pragma unroll
+        for (int u = 0; u < kIgStep; ++u) v[u] = row(cur[u].x);
+#pragma unroll
+        for (int u = 0; u < kIgStep; ++u) fma_acc(sum, __int_as_float(cur[u].y), v[u]);
+      }
+      acc[j] = sum;
+    }
+    // heavy inputs, a wave each: lanes take every 64th reference; their sum
+    // over the passes waits in gx
+    for (int h = wave; h < nh; h += kIgWaves) {
+      const int i = pm[a.IB - nh + h];
+      f32x4 sum = (f32x4)0.0f;
+      for (int k = s[i] + lane; k < s[i + 1]; k += 64) {
+        const int2 e = ent_heavy[k];
+        fma_acc(sum, __int_as_float(e.y), row(e.x));
+      }
+#pragma unroll
+      for (int d = 32; d > 0; d >>= 1)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) sum[v] += __shfl_xor(sum[v], d, 64);
+      if (lane < nb) {
+        float f = lane == 0 ? sum[0] : lane == 1 ? sum[1] : lane == 2 ? sum[2] : sum[3];
+        float* dst = gx + (int64_t)(b0 + lane) * a.IN + i0 + i;
+        if (p) f += *dst;
+        *dst = f;
+      }
+    }
+    __syncthreads();  // every read of the rows is done
+#pragma unroll
+    for (int j = 0; j < kIgSlots; ++j)
+      if (pv[j] >= 0) rows[pv[j] & 0xffff] = acc[j];
+    // heavy inputs' sums too: they may not be heavy in the next pass
+    for (int h = wave; h < nh; h += kIgWaves) {
+      const int i = pm[a.IB - nh + h];
+      if (lane < 4) {
+        float f = 0.0f;
+        if (lane < nb) f = gx[(int64_t)(b0 + lane) * a.IN + i0 + i];
+        reinterpret_cast<float*>(rows + i)[lane] = f;
+      }
+    }
+    __syncthreads();
+  }
+  for (int k = tid; k < n; k += kIgThreads) {
+    const f32x4 v = rows[k];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (u < nb) gx[(int64_t)(b0 + u) * a.IN + i0 + k] = v[u];
+  }
+}
+
+// ---------------------------------------------------------------------------
+// host side
+// ---------------------------------------------------------------------------
+static inline int64_t ig_round(int64_t n) { return (n + 3) & ~int64_t(3); }
+
+struct IgPlan {
+  IgArgs a;
+  int64_t keys, table, perm, slot, off, heavy, ent, ent_heavy, total;  // offsets, 4-byte words
+  int64_t groups, nkeys, tiles;
+};
+
+static IgPlan ig_plan(int64_t B, int64_t IN, int64_t OUT, int nsides, int K) {
+  IgPlan p{};
+  IgArgs& a = p.a;
+  a.B = (int)B; a.IN = (int)IN; a.OUT = (int)OUT; a.NS = nsides; a.K = K;
+  a.R2 = (int)(nsides * OUT);
+  a.R = nsides * OUT * (int64_t)K;
+  p.tiles = cdiv(std::max<int64_t>(B, 1), 4);
+  // a block of inputs per workgroup: all of them where the sample tiles fill
+  // the chip, else enough blocks to (each stages the rows again)
+  a.NB = (int)std::max<int64_t>(cdiv(IN, kIgBlock),
+                                std::min<int64_t>(cdiv(device_cus(), p.tiles), cdiv(IN, 256)));
+  a.IB = (int)(cdiv(cdiv(IN, a.NB), 64) * 64);
+  a.NB = (int)cdiv(IN, a.IB);
+  a.NP = (int)cdiv(a.R2, kIgRows);
+  a.RB = (int)(cdiv(cdiv(a.R2, a.NP), 4) * 4);
+  a.NP = (int)cdiv(a.R2, a.RB);
+  p.groups = (int64_t)a.NP * a.NB;
+  p.nkeys = p.groups * a.IB;
+  int64_t o = 0;
+  auto take = [&](int64_t n) {
+    const int64_t at = o;
+    o += ig_round(n);
+    return at;
+  };
+  p.keys = take(a.R);
+  p.table = take(ref_table_ints(a.R, p.nkeys));
+  p.perm = take(p.nkeys);
+  p.slot = take(p.nkeys);
+  p.off = take(p.groups * cdiv(a.IB, 64));
+  p.heavy = take(p.groups);
+  p.ent = take(2 * (a.R + p.groups * ig_slack(a.IB) + 3 * kIgStep * 64));  // read ahead
+  p.ent_heavy = take(2 * a.R);
+  p.total = o;
+  return p;
+}
+
+int64_t fc_input_grad_floats(int64_t B, int64_t IN, int64_t OUT, int nsides, int K) {
+  return ig_plan(B, IN, OUT, nsides, K).total;
+}
+
+int fc_input_grad(const float* gbr, int64_t B, int64_t IN, int64_t OUT, int nsides, int K,
+                  const int32_t* cand, const float* w, float* ws, float* gx, hipStream_t st) {
+  const IgPlan p = ig_plan(B, IN, OUT, nsides, K);
+  const IgArgs& a = p.a;
+  SLG_REQUIRE(a.R < (1LL << 31) && nsides * OUT < (1LL << 31) &&
+                  a.R + p.groups * ig_slack(a.IB) < (1LL << 31) && p.nkeys < (1LL << 31) &&
+                  p.tiles * a.NB < (1LL << 31),
+              SLG_E_SHAPE, "fc input gradient: too many references");
+  int* iw = reinterpret_cast<int*>(ws);
+  int *keys = iw + p.keys, *perm = iw + p.perm, *slot = iw + p.slot, *off = iw + p.off,
+      *heavy = iw + p.heavy;
+  int2* ent = reinterpret_cast<int2*>(iw + p.ent);
+  int2* ent_heavy = reinterpret_cast<int2*>(iw + p.ent_heavy);
+  const unsigned rb = (unsigned)cdiv(a.R, 256);
+  hipLaunchKernelGGL(ig_keys_kernel, dim3(rb), dim3(256), 0, st, a, cand, keys);
+  RefTable tb{};
+  const int rc = build_ref_table(keys, a.R, p.nkeys, iw + p.table, st, &tb);
+  if (rc) return rc;
+  hipLaunchKernelGGL(ig_slots_kernel, dim3((unsigned)p.groups), dim3(1024), 0, st, a, tb.start, perm,
+                     slot, off, heavy);
+  hipLaunchKernelGGL(ig_entries_kernel, dim3(rb), dim3(256), 0, st, a, tb.sorted, keys, tb.start, slot,
+                     off, w, ent, ent_heavy);
+  SLG_LAUNCH_CHECK("fc input gradient table");
+  const size_t lds = (size_t)std::max(a.RB + 1, a.IB) * 16;
+  if (lds > 65536) {
+    const hipError_t e = hipFuncSetAttribute((const void*)ig_gather_kernel,
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    SLG_REQUIRE(e == hipSuccess, (int)e, "fc input gradient: LDS %zu: %s", lds, hipGetErrorString(e));
+  }
+  hipLaunchKernelGGL(ig_gather_kernel, dim3((unsigned)(p.tiles * a.NB)), dim3(kIgThreads), lds, st, a,
+                     gbr, tb.start, perm, off, heavy, ent, ent_heavy, gx);
+  SLG_LAUNCH_CHECK("fc input gradient gather");
+  return 0;
+}
+
+}  // namespace slg

@@ -18,14 +18,10 @@
 //     output) operand gradient ga, gb to gbr [B][2*OUT] (coalesced rows).
 //   * fc_soft_bwd_reduce_kernel: sums the partials over sample ranges in
 //     ascending order.
-//   * the input gradient is the transposed problem: a table lists, for every
-//     input, the (row = side*OUT + o, weight) of the references to it in
-//     ascending reference order (count, scan, place, rank kernels); gbr is
-//     transposed to sample-minor rows gab [2*OUT][LB]; the gather kernel
-//     walks each input's entries with its lanes along samples.
+//   * the input gradient is a gather over a table of each input's references
+//     (fc_bwd_input.hip).
 #include "fc_soft_common.h"
 #include "fc_bwd_input.h"
-#include "ref_table.h"
 
 namespace slg {
 
@@ -97,162 +93,11 @@ __global__ void __launch_bounds__(256) fc_soft_pack_records_kernel(const int* __
 template <int KC>
 constexpr int bwd_threads() { return KC > 0 && KC <= 8 ? 1024 : 512; }
 
-// ---------------------------------------------------------------------------
-// Transposed reference table: for every input i, the references (o, side, k)
-// whose candidate is i, in ascending r = o*2K + side*K + k (a fixed order, so
-// the input gradient sums in the same order on every call), as entries
-// (row, weight) with row = side*OUT + o indexing the operand-gradient rows.
-// ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(256) fc_soft_bwd_keys_kernel(const int* __restrict__ cand, int R,
-                                                               int IN, int* __restrict__ keys) {
-  const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r < R) keys[r] = min(max(cand[r], 0), IN - 1);
-}
-
-__global__ void __launch_bounds__(256) fc_soft_bwd_entries_kernel(const int* __restrict__ sorted,
-                                                                  int R, int OUT, int NS, int K,
-                                                                  const float* __restrict__ w,
-                                                                  int2* __restrict__ ent) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= R) return;
-  const int r = sorted[j], SK = NS * K;  // r = (o * NS + side) * K + k
-  const int o = r / SK, side = (r - o * SK) / K;
-  ent[j] = make_int2(side * OUT + o, __float_as_int(w[r]));
-}
-
-// gab [R2][LB] = transpose of gbr [B][R2] (rows b >= B of gab's columns are
-// zero), through a 64 x 64 LDS tile; float4 loads along gbr rows when R2 is
-// a multiple of 4, float4 stores along gab rows (LB is a multiple of 64).
-__global__ void __launch_bounds__(256) fc_soft_bwd_transpose_kernel(const float* __restrict__ gbr,
-                                                                    int B, int R2, int64_t LB,
-                                                                    int n_rtiles,
-                                                                    float* __restrict__ gab) {
-  __shared__ float t[64][65];  // [b][r]
-  const int rt = blockIdx.x % n_rtiles, bt = blockIdx.x / n_rtiles;
-  const int r0 = rt * 64, b0 = bt * 64;
-  const int c4 = threadIdx.x & 15, q = threadIdx.x >> 4;  // 16 float4 columns x 16 rows
-  if ((R2 & 3) == 0) {
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const int bl = q + 16 * k, b = b0 + bl, r = r0 + 4 * c4;
-      float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-      if (b < B && r < R2) v = *reinterpret_cast<const float4*>(gbr + (int64_t)b * R2 + r);
-      t[bl][4 * c4] = v.x;
-      t[bl][4 * c4 + 1] = v.y;
-      t[bl][4 * c4 + 2] = v.z;
-      t[bl][4 * c4 + 3] = v.w;
-    }
-  } else {
-    const int c = threadIdx.x & 63, qq = threadIdx.x >> 6;
-#pragma unroll
-    for (int k = 0; k < 16; ++k) {
-      const int bl = qq + 4 * k, b = b0 + bl, r = r0 + c;
-      t[bl][c] = (b < B && r < R2) ? gbr[(int64_t)b * R2 + r] : 0.0f;
-    }
-  }
-  __syncthreads();
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const int rl = q + 16 * k, r = r0 + rl;
-    if (r < R2) {
-      const float4 v = make_float4(t[4 * c4][rl], t[4 * c4 + 1][rl], t[4 * c4 + 2][rl],
-                                   t[4 * c4 + 3][rl]);
-      *reinterpret_cast<float4*>(gab + (int64_t)r * LB + b0 + 4 * c4) = v;
-    }
-  }
-}
-
-// Input gradient from the node-gradient rows gab [2*OUT][LB] (row side*OUT+o,
-// sample-minor): gx[b][i] = sum over the entries e of input i, in table
-// order, of weight(e) * gab[row(e)][b]. A workgroup owns 4*IW inputs x 64*V
-// samples. Each wave walks the entries of its IW consecutive inputs as one
-// flat range (contiguous in the table) with its lanes along samples: the
-// entries are wave-uniform (scalar loads, the next 8 prefetched), each costs
-// one coalesced 64V-sample row-segment load, and 8 such loads are in flight.
-// An input's sum is complete when the walk reaches the next input's start.
-// The results go through LDS so gx rows are written contiguously.
-template <int V, int IW>
-__global__ void __launch_bounds__(256) fc_soft_bwd_gather_kernel(const float* __restrict__ gab,
-                                                                 int64_t LB, int B, int IN,
-                                                                 const int* __restrict__ start,
-                                                                 const int2* __restrict__ ent,
-                                                                 int n_itiles, int n_blocks,
-                                                                 float* __restrict__ gx) {
-  using vt = typename vecf<V>::t;
-  constexpr int NI = 4 * IW;       // inputs per workgroup
-  constexpr int NS = 64 * V;       // samples per workgroup
-  constexpr int G = 8;             // entries per step
-  __shared__ float T[NI][NS + 1];  // [input][sample]
-  const int L = (int)xcd_logical_id(blockIdx.x, gridDim.x);
-  if (L >= n_blocks) return;
-  const int it = L % n_itiles, sc = L / n_itiles;
-  const int i0 = it * NI;
-  const int b0 = sc * NS;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  const float* col = gab + b0 + lane * V;
-  const int ia = i0 + wave * IW;
-  const int iend = min(ia + IW, IN);
-  int cur = ia;  // input whose sum is being accumulated
-  float acc[V];
-#pragma unroll
-  for (int v = 0; v < V; ++v) acc[v] = 0.0f;
-  if (ia < iend) {
-    int e = start[ia];
-    const int e_end = start[iend];
-    int nb = start[ia + 1];  // first entry of input cur + 1
-    int2 qn[G];
-#pragma unroll
-    for (int u = 0; u < G; ++u) qn[u] = ent[min(e + u, max(e_end - 1, 0))];
-    while (e < e_end) {
-      int2 q[G];
-#pragma unroll
-      for (int u = 0; u < G; ++u) q[u] = qn[u];
-      vt g[G];
-#pragma unroll
-      for (int u = 0; u < G; ++u) g[u] = *reinterpret_cast<const vt*>(col + (int64_t)q[u].x * LB);
-      const int en = e + G;
-#pragma unroll
-      for (int u = 0; u < G; ++u) qn[u] = ent[min(en + u, e_end - 1)];
-#pragma unroll
-      for (int u = 0; u < G; ++u) {
-        if (e + u < e_end) {
-          while (e + u == nb) {  // input cur is complete (inputs without entries: zero)
-#pragma unroll
-            for (int v = 0; v < V; ++v) {
-              T[cur - i0][lane * V + v] = acc[v];
-              acc[v] = 0.0f;
-            }
-            ++cur;
-            nb = start[cur + 1];
-          }
-#pragma unroll
-          for (int v = 0; v < V; ++v) acc[v] = fmaf(__int_as_float(q[u].y), lanev(g[u], v), acc[v]);
-        }
-      }
-      e = en;
-    }
-  }
-  for (; cur < ia + IW; ++cur) {  // the last input with entries, then empty ones
-#pragma unroll
-    for (int v = 0; v < V; ++v) {
-      T[cur - i0][lane * V + v] = acc[v];
-      acc[v] = 0.0f;
-    }
-  }
-  __syncthreads();
-  const int c = threadIdx.x % NI;
-#pragma unroll 4
-  for (int s = threadIdx.x / NI; s < NS; s += 256 / NI) {
-    if (b0 + s < B && i0 + c < IN) gx[(int64_t)(b0 + s) * IN + i0 + c] = T[c][s];
-  }
-}
-
 // Weight / node-parameter gradient partials of one output per thread over a
 // range of sample tiles: part [NR][2K+4][OUT] (components w_a[0..K),
 // w_b[0..K), param[0..4)); with gbr, also the node's operand gradients
 // ga, gb of every (sample, output) at gbr[b][o], gbr[b][OUT+o] (rows of
-// 2*OUT, coalesced along the outputs), transposed for the gather kernel.
+// 2*OUT, coalesced along the outputs).
 //
 // WIDE (rows wider than LDS): one sample per tile, staged slab by slab (SL
 // inputs at a time); each thread keeps its output's 2K gathered operands in
@@ -338,7 +183,7 @@ fc_soft_bwd_w_kernel(const float* __restrict__ x, int B, int IN, int OUT, int Kr
 #pragma unroll
       for (int q = 0; q < 4; ++q) sp[q] += gp[q];
     }
-    if (gbr != nullptr && valid) {  // sample rows of 2*OUT; tiles end at or before LB
+    if (gbr != nullptr && valid) {  // sample rows of 2*OUT
 #pragma unroll
       for (int s = 0; s < S; ++s) {
         gbr[(int64_t)(b0 + s) * (2 * OUT) + o] = ga[s];
@@ -411,11 +256,6 @@ static int bwd_tile(int64_t IN, int64_t per_float_bytes_per_sample) {
   return 0;
 }
 
-constexpr int kGatherV = 4;              // samples per lane in the gather kernel
-constexpr int kGatherIW = 8;             // inputs per wave in the gather kernel
-constexpr int kGatherSamples = 64 * kGatherV;
-constexpr int kGatherInputs = 4 * kGatherIW;
-
 inline int64_t round4(int64_t n) { return (n + 3) & ~int64_t(3); }
 
 // Workspace (in 4-byte words): records | partials | gbr | input-gradient part.
@@ -426,63 +266,6 @@ struct BwdPlan {
   int64_t rec_floats, part_floats, gbr_floats, in_floats;
   int64_t total() const { return rec_floats + part_floats + gbr_floats + in_floats; }
 };
-
-// Input-gradient workspace: gab [nsides*OUT][LB] | keys | table | entries.
-struct InPlan {
-  int64_t LB, R, gab_floats, keys_ints, table_ints, ent_ints;
-  int64_t total() const { return gab_floats + keys_ints + table_ints + ent_ints; }
-};
-
-static InPlan in_plan(int64_t B, int64_t IN, int64_t OUT, int nsides, int K) {
-  InPlan q{};
-  q.LB = cdiv(std::max<int64_t>(B, 1), kGatherSamples) * kGatherSamples;
-  q.R = nsides * OUT * (int64_t)K;
-  q.gab_floats = nsides * OUT * q.LB;
-  q.keys_ints = round4(q.R);
-  q.table_ints = ref_table_ints(q.R, IN);
-  q.ent_ints = 2 * q.R;
-  return q;
-}
-
-int64_t fc_input_grad_floats(int64_t B, int64_t IN, int64_t OUT, int nsides, int K) {
-  return in_plan(B, IN, OUT, nsides, K).total();
-}
-
-int fc_input_grad(const float* gbr, int64_t B, int64_t IN, int64_t OUT, int nsides, int K,
-                  const int32_t* cand, const float* w, float* ws, float* gx, hipStream_t st) {
-  const InPlan q = in_plan(B, IN, OUT, nsides, K);
-  SLG_REQUIRE(q.R < (1LL << 31) && nsides * OUT < (1LL << 31), SLG_E_SHAPE,
-              "fc input gradient: too many references");
-  float* gab = ws;
-  int* keys = reinterpret_cast<int*>(gab + q.gab_floats);
-  int* table = keys + q.keys_ints;
-  int2* ent = reinterpret_cast<int2*>(table + q.table_ints);  // 8-byte aligned: offsets are even
-  const int R = (int)q.R;
-  hipLaunchKernelGGL(fc_soft_bwd_keys_kernel, dim3((unsigned)cdiv(R, 256)), dim3(256), 0, st,
-                     cand, R, (int)IN, keys);
-  RefTable tb{};
-  int rc = build_ref_table(keys, R, IN, table, st, &tb);
-  if (rc) return rc;
-  hipLaunchKernelGGL(fc_soft_bwd_entries_kernel, dim3((unsigned)cdiv(R, 256)), dim3(256), 0, st,
-                     tb.sorted, R, (int)OUT, nsides, K, w, ent);
-  SLG_LAUNCH_CHECK("fc input gradient entries");
-  const int R2 = (int)(nsides * OUT);
-  const int n_rtiles = (int)cdiv(R2, 64);
-  const int64_t n_tr = n_rtiles * (q.LB / 64);
-  SLG_REQUIRE(n_tr < (1LL << 31), SLG_E_SHAPE, "fc input gradient: grid too large");
-  hipLaunchKernelGGL(fc_soft_bwd_transpose_kernel, dim3((unsigned)n_tr), dim3(256), 0, st, gbr,
-                     (int)B, R2, q.LB, n_rtiles, gab);
-  SLG_LAUNCH_CHECK("fc input gradient transpose");
-  const int n_itiles = (int)cdiv(IN, kGatherInputs);
-  const int64_t n_blocks = n_itiles * (q.LB / kGatherSamples);
-  SLG_REQUIRE(n_blocks < (1LL << 31) - 8, SLG_E_SHAPE, "fc input gradient: grid too large");
-  const int64_t grid = cdiv(n_blocks, 8) * 8;  // a multiple of 8 for the XCD remap
-  auto gather = fc_soft_bwd_gather_kernel<kGatherV, kGatherIW>;
-  hipLaunchKernelGGL(gather, dim3((unsigned)grid), dim3(256), 0, st, gab, q.LB, (int)B, (int)IN,
-                     tb.start, ent, n_itiles, (int)n_blocks, gx);
-  SLG_LAUNCH_CHECK("fc input gradient gather");
-  return 0;
-}
 
 static BwdPlan bwd_plan(int64_t B, int64_t IN, int64_t OUT, int K) {
   BwdPlan p{};
@@ -504,10 +287,9 @@ static BwdPlan bwd_plan(int64_t B, int64_t IN, int64_t OUT, int K) {
   p.NR = (int)std::max<int64_t>(1, std::min<int64_t>(n_tiles, slots / p.n_orange));
   p.tiles_per_range = (int)cdiv(n_tiles, p.NR);
   p.NR = (int)cdiv(n_tiles, p.tiles_per_range);
-  const int64_t LB = cdiv(std::max<int64_t>(B, 1), kGatherSamples) * kGatherSamples;
   p.rec_floats = p.SL ? 0 : cdiv(OUT, 64) * 64 * (int64_t)rec_quads(K) * 4;
   p.part_floats = round4((int64_t)p.NR * (2 * K + 4) * OUT);
-  p.gbr_floats = 2 * OUT * LB;  // rows b < n_tiles * Sw <= LB
+  p.gbr_floats = round4(2 * OUT * n_tiles * p.Sw);  // the last tile's rows whole
   p.in_floats = fc_input_grad_floats(B, IN, OUT, 2, K);
   return p;
 }

@@ -16,33 +16,57 @@ __global__ void __launch_bounds__(256) ref_count_kernel(const int* __restrict__ 
   if (r < R) atomicAdd(&cnt[keys[r]], 1);
 }
 
-// One workgroup: start[0..n] = exclusive scan of cnt, cursor = start. cnt
-// and cursor may be the same array: each element is read before it is
-// written, by the one thread that owns it.
+// One workgroup: start[0..n] = exclusive scan of cnt, cursor = start, 4096
+// counts a step (coalesced: 20000 counts took 13 us with a run of counts per
+// thread). cnt and cursor may be the same array: each element is read before
+// it is written, by the one thread that owns it.
 __global__ void __launch_bounds__(1024) ref_scan_kernel(const int* cnt, int n,
                                                         int* __restrict__ start, int* cursor) {
-  __shared__ int part[1024];
-  const int t = threadIdx.x;
-  const int per = (n + 1023) / 1024;
-  const int lo = min(t * per, n), hi = min(lo + per, n);
-  int sum = 0;
-  for (int i = lo; i < hi; ++i) sum += cnt[i];
-  part[t] = sum;
-  __syncthreads();
-  for (int d = 1; d < 1024; d <<= 1) {  // inclusive Hillis-Steele scan
-    const int v = t >= d ? part[t - d] : 0;
+  __shared__ int part[16];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  int run = 0;
+  auto load = [&](int base, int (&c)[4]) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int i = base + 4 * t + u;
+      c[u] = i < n ? cnt[i] : 0;
+    }
+  };
+  int c[4], nx[4];
+  load(0, nx);
+  for (int base = 0; base < n; base += 4096) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) c[u] = nx[u];
+    if (base + 4096 < n) load(base + 4096, nx);  // the next step's counts in flight
+    int sum = c[0] + c[1] + c[2] + c[3];
+    int x = sum;  // inclusive over the wave
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int y = __shfl_up(x, d, 64);
+      if (lane >= d) x += y;
+    }
+    if (lane == 63) part[wave] = x;
     __syncthreads();
-    part[t] += v;
+    int before = 0, all = 0;
+#pragma unroll
+    for (int w = 0; w < 16; ++w) {
+      before += w < wave ? part[w] : 0;
+      all += part[w];
+    }
+    int at = run + before + x - sum;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int i = base + 4 * t + u;
+      if (i < n) {
+        start[i] = at;
+        cursor[i] = at;
+      }
+      at += c[u];
+    }
+    run += all;
     __syncthreads();
   }
-  int run = part[t] - sum;
-  for (int i = lo; i < hi; ++i) {
-    const int c = cnt[i];
-    start[i] = run;
-    cursor[i] = run;
-    run += c;
-  }
-  if (t == 1023) start[n] = part[1023];
+  if (t == 0) start[n] = run;
 }
 
 __global__ void __launch_bounds__(256) ref_fill_kernel(const int* __restrict__ keys, int R,
