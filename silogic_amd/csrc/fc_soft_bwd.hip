@@ -90,6 +90,7 @@ __global__ void __launch_bounds__(256) fc_soft_pack_records_kernel(const int* __
   rec[t] = v;
 }
 
+constexpr int kBwdAheadQuads = 3;
 template <int KC>
 constexpr int bwd_threads() { return KC > 0 && KC <= 8 ? 1024 : 512; }
 
@@ -103,10 +104,11 @@ constexpr int bwd_threads() { return KC > 0 && KC <= 8 ? 1024 : 512; }
 // inputs at a time); each thread keeps its output's 2K gathered operands in
 // registers, filling those in the current slab, then runs the same math.
 // Parameters come from the separate arrays (32-bit indices).
-template <int NODE, int KC, int S, bool WIDE>
+template <int NODE, int KC, int S, bool WIDE, bool AHEAD>
 __global__ void __launch_bounds__((bwd_threads<KC>()))
 fc_soft_bwd_w_kernel(const float* __restrict__ x, int B, int IN, int OUT, int Kr, ParamView pv,
-                     float inv_tau, const float* __restrict__ gy, int n_orange, int tiles_per_range,
+                     float inv_tau, const float* __restrict__ gy, int n_orange, int n_range,
+                     int tiles_per_range,
                      float* __restrict__ part, float* __restrict__ gbr, int SL) {
   static_assert(!WIDE || S == 1, "slab staging takes one sample per tile");
   constexpr int KM = KC > 0 ? KC : 16;
@@ -114,8 +116,12 @@ fc_soft_bwd_w_kernel(const float* __restrict__ x, int B, int IN, int OUT, int Kr
   extern __shared__ __align__(16) unsigned char smem[];
   vt* xs = reinterpret_cast<vt*>(smem);
   const int K = KC > 0 ? KC : Kr;
-  const int r_o = (int)(blockIdx.x % (uint32_t)n_orange);
-  const int r_b = (int)(blockIdx.x / (uint32_t)n_orange);
+  // the output ranges of one sample range on one XCD: they stage the same
+  // rows, which then cross the fabric once
+  const uint32_t lid = xcd_logical_id(blockIdx.x, gridDim.x);
+  const int r_o = (int)(lid % (uint32_t)n_orange);
+  const int r_b = (int)(lid / (uint32_t)n_orange);
+  if (r_b >= n_range) return;  // the grid is padded to a multiple of 8
   const int o = r_o * blockDim.x + threadIdx.x;
   const bool valid = o < OUT;
   FcParams<KM> P;
@@ -126,6 +132,13 @@ fc_soft_bwd_w_kernel(const float* __restrict__ x, int B, int IN, int OUT, int Kr
     P.ia[k] = (int)min((uint32_t)P.ia[k], lim);
     P.ib[k] = (int)min((uint32_t)P.ib[k], lim);
   }
+  // one register per index pair (inputs below 65536), unpacked where it is
+  // used: the registers go to the next tile's rows
+  uint32_t pk[WIDE ? 1 : KM];
+  if constexpr (!WIDE) {
+#pragma unroll
+    for (int k = 0; k < KM; ++k) pk[k] = (uint32_t)P.ia[k] | ((uint32_t)P.ib[k] << 16);
+  }
   const int* ia = P.ia;
   const int* ib = P.ib;
   float swa[KM], swb[KM], sp[4] = {0.f, 0.f, 0.f, 0.f};
@@ -134,9 +147,64 @@ fc_soft_bwd_w_kernel(const float* __restrict__ x, int B, int IN, int OUT, int Kr
 
   const int n_tiles = (B + S - 1) / S;
   const int t_end = min(n_tiles, (r_b + 1) * tiles_per_range);
+  // AHEAD: the next tile's rows (up to NPF quads of inputs per thread) ride in
+  // registers while this tile computes: staged between two barriers with
+  // nothing else in flight, three quarters of the wave cycles waited (10000 ->
+  // 10000, K = 8, B = 4096: 386 -> 318 us; a workgroup with one tile has
+  // nothing to overlap, 12.0 against 13.7 us at 2000 -> 2000, B = 256).
+  constexpr int NPF = AHEAD ? kBwdAheadQuads : 0;
+  const int n4 = IN >> 2, T = blockDim.x;
+  float4 pf[NPF > 0 ? NPF : 1][S];
+  // rows through buffer resources: one vector offset for all loads, zeros
+  // past a row's end (and, by a size of 0, past the batch)
+  const int vq = threadIdx.x * 16, vo = valid ? o * 4 : 0x7ffffffc;
+  auto row_of = [&](const float* p, int64_t stride, int b, int64_t n) {
+    return uniform_rsrc(p + (int64_t)min(b, B - 1) * stride, b < B ? (int)(n * 4) : 0);
+  };
+  auto issue = [&](int b0) {
+#pragma unroll
+    for (int v = 0; v < S; ++v) {
+      const auto xr = row_of(x, IN, b0 + v, IN);
+#pragma unroll
+      for (int u = 0; u < NPF; ++u)
+        pf[u][v] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(xr, vq + u * T * 16, 0, 0));
+    }
+  };
+  auto place = [&]() {
+#pragma unroll
+    for (int u = 0; u < NPF; ++u) {
+      const int q = threadIdx.x + u * T;
+      if (q < n4) {
+#pragma unroll
+        for (int cc = 0; cc < 4; ++cc) {
+          float e[S];
+#pragma unroll
+          for (int v = 0; v < S; ++v) e[v] = lanev(pf[u][v], cc);
+          xs[4 * q + cc] = make_vec<S>(e);
+        }
+      }
+    }
+  };
+  auto load_g = [&](int b0, float (&g)[S]) {
+#pragma unroll
+    for (int v = 0; v < S; ++v)
+      g[v] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(row_of(gy, OUT, b0 + v, OUT), vo, 0, 0));
+  };
+  float gn[S];
+  if (r_b * tiles_per_range < t_end) {
+    load_g(r_b * tiles_per_range * S, gn);
+    if constexpr (AHEAD) {
+      issue(r_b * tiles_per_range * S);
+      place();
+      __syncthreads();
+    }
+  }
   for (int t = r_b * tiles_per_range; t < t_end; ++t) {
     const int b0 = t * S;
-    vt xa[WIDE ? KM : 1], xb[WIDE ? KM : 1];  // wide: the gathered operands
+    float g[S];
+#pragma unroll
+    for (int v = 0; v < S; ++v) g[v] = gn[v];
+    vt xa[KM], xb[KM];  // the gathered operands
     if constexpr (WIDE) {
 #pragma unroll
       for (int k = 0; k < KM; ++k) xa[k] = xb[k] = 0.0f;
@@ -155,52 +223,80 @@ fc_soft_bwd_w_kernel(const float* __restrict__ x, int B, int IN, int OUT, int Kr
           }
         }
       }
-    } else {
+    } else if constexpr (!AHEAD) {
       __syncthreads();  // the previous tile's reads are done
       stage_rows<S, false>(xs, x, B, IN, b0);  // the other output ranges re-read these rows
       __syncthreads();
     }
-    auto opa = [&](int k) -> vt {
-      if constexpr (WIDE) return xa[k]; else return xs[ia[k]];
-    };
-    auto opb = [&](int k) -> vt {
-      if constexpr (WIDE) return xb[k]; else return xs[ib[k]];
+    if (t + 1 < t_end) {
+      if constexpr (AHEAD) issue(b0 + S);
+      load_g(b0 + S, gn);
+    }
+    // operands kept from the sums to the weight gradients where the registers
+    // hold them, else gathered again, four candidates at a time
+    constexpr bool kHold = WIDE || KC == 4 || 2 * KM * S <= 16;
+    constexpr int GK = kHold ? KM : 4;
+    auto gather = [&](int k0) {
+#pragma unroll
+      for (int k = k0; k < k0 + GK; ++k) {
+        if (KC > 0 || k < K) {
+          asm volatile("" : "+v"(pk[WIDE ? 0 : k]));  // no unpacked copies across the loop
+          xa[k] = xs[pk[WIDE ? 0 : k] & 0xffffu];
+          xb[k] = xs[pk[WIDE ? 0 : k] >> 16];
+        }
+      }
+      if constexpr (!kHold) __builtin_amdgcn_sched_barrier(0);
     };
     vt A = zero_vec<vt>(), Bv = zero_vec<vt>();
 #pragma unroll
-    for (int k = 0; k < KM; ++k) {
-      if (KC > 0 || k < K) {
-        fma_acc(A, P.fa[k], opa(k));
-        fma_acc(Bv, P.fb[k], opb(k));
+    for (int k0 = 0; k0 < KM; k0 += GK) {
+      if constexpr (!WIDE) gather(k0);
+#pragma unroll
+      for (int k = k0; k < k0 + GK; ++k) {
+        if (KC > 0 || k < K) {
+          fma_acc(A, P.fa[k], xa[k]);
+          fma_acc(Bv, P.fb[k], xb[k]);
+        }
       }
+      if constexpr (!kHold) __builtin_amdgcn_sched_barrier(0);
     }
     float ga[S], gb[S];
 #pragma unroll
     for (int s = 0; s < S; ++s) {
-      const float g = (valid && b0 + s < B) ? gy[(int64_t)(b0 + s) * OUT + o] : 0.0f;
       float gp[4];
-      node_grad<NODE>(lanev(A, s), lanev(Bv, s), g, P.p, inv_tau, ga[s], gb[s], gp);
+      node_grad<NODE>(lanev(A, s), lanev(Bv, s), g[s], P.p, inv_tau, ga[s], gb[s], gp);
 #pragma unroll
       for (int q = 0; q < 4; ++q) sp[q] += gp[q];
     }
-    if (gbr != nullptr && valid) {  // sample rows of 2*OUT
+    if (gbr != nullptr) {  // sample rows of 2*OUT; outputs past OUT are not stored
 #pragma unroll
       for (int s = 0; s < S; ++s) {
-        gbr[(int64_t)(b0 + s) * (2 * OUT) + o] = ga[s];
-        gbr[(int64_t)(b0 + s) * (2 * OUT) + OUT + o] = gb[s];
+        const auto gr = uniform_rsrc(gbr + (int64_t)(b0 + s) * (2 * OUT), OUT * 8);
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(ga[s]), gr, vo, 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(gb[s]), gr, valid ? vo + OUT * 4 : vo, 0, 0);
       }
     }
     // second pass over the candidates: sum_s ga[s] * x[s][cand]
+    if constexpr (!kHold) asm volatile("" ::: "memory");  // not the first pass's values
 #pragma unroll
-    for (int k = 0; k < KM; ++k) {
-      if (KC > 0 || k < K) {
-        const vt va = opa(k), vb = opb(k);
+    for (int k0 = 0; k0 < KM; k0 += GK) {
+      if constexpr (!kHold) gather(k0);
 #pragma unroll
-        for (int s = 0; s < S; ++s) {
-          swa[k] = fmaf(ga[s], lanev(va, s), swa[k]);
-          swb[k] = fmaf(gb[s], lanev(vb, s), swb[k]);
+      for (int k = k0; k < k0 + GK; ++k) {
+        if (KC > 0 || k < K) {
+#pragma unroll
+          for (int s = 0; s < S; ++s) {
+            swa[k] = fmaf(ga[s], lanev(xa[k], s), swa[k]);
+            swb[k] = fmaf(gb[s], lanev(xb[k], s), swb[k]);
+          }
         }
       }
+      if constexpr (!kHold) __builtin_amdgcn_sched_barrier(0);
+    }
+    if constexpr (AHEAD) {
+      __syncthreads();  // this tile's reads are done
+      if (t + 1 < t_end) place();
+      __syncthreads();
     }
   }
   if (part != nullptr && valid) {
@@ -277,7 +373,7 @@ static BwdPlan bwd_plan(int64_t B, int64_t IN, int64_t OUT, int K) {
   }
   const int threads = K == 8 || K == 4 ? 1024 : 512;
   p.n_orange = (int)cdiv(OUT, threads);
-  const int64_t n_tiles = p.Sw ? cdiv(std::max<int64_t>(B, 1), p.Sw) : 1;
+  const int64_t n_tiles = cdiv(std::max<int64_t>(B, 1), p.Sw);
   // one round of workgroups: as many sample ranges as resident slots allow
   // (2048 threads and 160 KB of LDS per CU); a partial second round would
   // double the kernel's time
@@ -298,7 +394,13 @@ template <int NODE, int KC, int S, bool WIDE = false>
 static int launch_bwd_w(const float* x, int64_t B, int64_t IN, int64_t OUT, int K,
                         const ParamView& pv, float inv_tau, const float* gy, const BwdPlan& p,
                         float* part, float* gbr, hipStream_t st) {
-  auto kern = fc_soft_bwd_w_kernel<NODE, KC, S, WIDE>;
+  auto kern = fc_soft_bwd_w_kernel<NODE, KC, S, WIDE, false>;
+  if constexpr (!WIDE && S <= 2) {
+    // rows of whole quads that the workgroup's registers hold a tile of
+    if (p.tiles_per_range > 1 && IN % 4 == 0 && IN / 4 <= kBwdAheadQuads * bwd_threads<KC>() &&
+        (uintptr_t)x % 16 == 0)
+      kern = fc_soft_bwd_w_kernel<NODE, KC, S, WIDE, true>;
+  }
   const size_t lds = WIDE ? (size_t)p.SL * 4 : (size_t)IN * S * 4;
   if (lds > 65536) {
     hipError_t e = hipFuncSetAttribute((const void*)kern,
@@ -308,8 +410,8 @@ static int launch_bwd_w(const float* x, int64_t B, int64_t IN, int64_t OUT, int 
       return (int)e;
     }
   }
-  hipLaunchKernelGGL(kern, dim3((unsigned)(p.n_orange * p.NR)), dim3(bwd_threads<KC>()), lds, st,
-                     x, (int)B, (int)IN, (int)OUT, K, pv, inv_tau, gy, p.n_orange,
+  hipLaunchKernelGGL(kern, dim3((unsigned)(cdiv(p.n_orange * p.NR, 8) * 8)), dim3(bwd_threads<KC>()), lds, st,
+                     x, (int)B, (int)IN, (int)OUT, K, pv, inv_tau, gy, p.n_orange, p.NR,
                      p.tiles_per_range, part, gbr, p.SL);
   SLG_LAUNCH_CHECK("fc_soft_bwd_w");
   return 0;
