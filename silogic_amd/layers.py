@@ -8,9 +8,11 @@ Compute runs on the HIP kernels of ``libsilogic_hip.so``:
 * ``LogicLayer.forward`` -> Top-K gather + node. Without gradients the
   parameters (``softmax(conn)``, node coefficients, clamped indices) are
   packed into one record per output by ``slg_fc_soft_records`` and the layer
-  runs on ``slg_fc_soft_fwd_records``; with gradients they come from
-  differentiable torch ops (the reference's ``_fused`` split,
-  layers.py:111-123) and the layer runs on ``slg_fc_soft_fwd``.
+  runs on ``slg_fc_soft_fwd_records``; with gradients and a plain softmax
+  selection they come from ``slg_layer_params`` inside the layer's operator
+  (its backward ends in ``slg_layer_params_bwd``), else from differentiable
+  torch ops (the reference's ``_fused`` split, layers.py:111-123), and the
+  layer runs on ``slg_fc_soft_fwd``.
 * ``LogicLayer.forward_hard`` -> pack, one packed layer, unpack.
 * ``ConvLogicTree.forward`` -> ``slg_conv_soft_fwd``; networks call
   ``forward_pooled``, which fuses the following ``OrPool``.
@@ -133,6 +135,13 @@ class LogicLayer(nn.Module):
                                    conn.k)
         return cand, w, npar
 
+    def _params_op(self, raw):
+        """Whether the layer trains on the operators that take its own
+        parameters (``slg_layer_params``): a plain softmax selection."""
+        conn = self._conn
+        return (self.node.plain_softmax() and not getattr(conn, "ste", False)
+                and ops.param_levels_ok(getattr(conn, "conn", None), [raw], conn.k))
+
     def records_ok(self):
         """Whether the forward without gradients runs on per-output records:
         a plain softmax selection over inputs below 65536 (records hold 16-bit
@@ -194,10 +203,21 @@ class LogicLayer(nn.Module):
                 z = ops.fc_lut_soft(x, conn.candidates_i32(), conn.weights(),
                                     self.node.corner_z(), False)
                 return torch.sigmoid(z * self.node.inv_tau)
+            # fixed wiring has one sigmoid to fuse, which torch launches faster
+            if (_needs_grad(self, x) and not isinstance(conn, FixedConnectome)
+                    and self._params_op(self.node.logits)):
+                return torch.ops.silogic_hip.fc_lut_layer(
+                    x, conn.candidates_i32(), conn.conn, self.node.logits,
+                    bool(self.node.hybrid))[0]
             return ops.fc_lut_soft(x, conn.candidates_i32(), conn.weights(),
                                    torch.sigmoid(self.node.logits), self.node.hybrid)
         self._check_supported()
         grad = _needs_grad(self, x)
+        if grad and self._params_op(self.node.raw()):
+            conn = self._conn
+            return torch.ops.silogic_hip.fc_layer(
+                x, conn.candidates_i32(), getattr(conn, "conn", None), self.node.raw(),
+                self.node.kind, float(self._inv_tau()))[0]
         if not grad and self.records_ok():
             K = self.n_candidates
             rec = derived.cached(self, "_derived_records", (derived.state_key(self), K),
@@ -521,7 +541,23 @@ class ConvLogicTree(nn.Module):
             rec = self.soft_records(x.shape[1:], pool)
             return ops.conv_soft_rec(x, rec, self.n, self._kind(), self.d, self.node_arity, K,
                                      self.padding, pool)
-        w, npar = self.soft_params(_needs_grad(self, x))
+        grad = _needs_grad(self, x)
+        if grad and self._plain_soft():
+            conn = None if self.connect == "fixed" else self.conn
+            if self.node_name == "gate16":
+                levels = list(self.gate_logits)
+            else:
+                levels = [nd.raw() for nd in self.tree_nodes]
+            # the sizes slg_conv_soft_bwd takes (others: the composite backward)
+            sizes = K <= 8 and max(x.shape[1], self.n) < 1 << 20 and max(x.shape[2:]) < 4096
+            if sizes and ops.param_levels_ok(conn, levels, K):
+                gate16 = self.node_name == "gate16"
+                levels = levels + [None] * (5 - len(levels))
+                return torch.ops.silogic_hip.conv_layer(
+                    x, conn, *levels, self.basis if gate16 else None, cm, ch, cw, self._kind(),
+                    self.d, self.node_arity, K, self.padding, bool(pool),
+                    1.0 / self.tau if self.node_name == "walsh" else 1.0)[0]
+        w, npar = self.soft_params(grad)
         return ops.conv_soft(x, npar, w, cm, ch, cw, self._kind(), self.d, self.node_arity, K,
                              self.padding, pool)
 

@@ -14,7 +14,7 @@ Gradients an op does not need come back from the backward ops as empty
 ``[0]`` tensors (a custom op returns tensors, not None) and are turned into
 None before autograd sees them.
 """
-from typing import List, Tuple
+from typing import List, Optional, Tuple
 
 import torch
 from torch import Tensor
@@ -204,6 +204,123 @@ orpool.register_autograd(_orpool_backward, setup_context=_orpool_setup)
 
 
 # ---------------------------------------------------------------------------
+# Layers from their own parameters: the training forms of the modules. Each
+# op also returns the weights and node parameters it derived (saved for its
+# backward; not differentiable themselves).
+# ---------------------------------------------------------------------------
+def _layer_outputs(x, y_shape, w_shape, np_shape):
+    return tuple(x.new_empty(s, dtype=torch.float32) for s in (y_shape, w_shape, np_shape))
+
+
+@torch.library.custom_op(f"{_NS}::fc_layer", mutates_args=())
+def fc_layer(x: Tensor, cand: Tensor, conn: Optional[Tensor], raw: Tensor, node_kind: int,
+             inv_tau: float) -> Tuple[Tensor, Tensor, Tensor]:
+    """Gate layer: ``x [B,IN]``, ``cand/conn [OUT,A,K]``, ``raw`` the node's
+    parameters -> ``(y [B,OUT], w [OUT,A,K], npar)``. ``A = 2`` gate16 and
+    walsh nodes, and arity-2 multilinear ones, as ``fc_soft``."""
+    ops.require_gpu(x, cand, conn, raw)
+    cand = ops._c(cand, torch.int32)
+    w, npar = ops.layer_params(conn, tuple(cand.shape), [raw], node_kind, 2)
+    npar = npar.view(-1, 4)
+    return ops._fc_soft_launch(ops._as_f32(x), cand, w, npar, node_kind, inv_tau), w, npar
+
+
+@fc_layer.register_fake
+def _(x, cand, conn, raw, node_kind, inv_tau):
+    return _layer_outputs(x, (x.shape[0], cand.shape[0]), cand.shape, (cand.shape[0], 4))
+
+
+@torch.library.custom_op(f"{_NS}::fc_layer_bwd", mutates_args=())
+def fc_layer_bwd(x: Tensor, cand: Tensor, raw: Tensor, w: Tensor, npar: Tensor, node_kind: int,
+                 inv_tau: float, gy: Tensor, need_x: bool, need_conn: bool,
+                 need_raw: bool) -> Tuple[Tensor, Tensor, Tensor]:
+    """``(gx, gconn, graw)`` of fc_layer; unneeded ones are empty."""
+    gx, gw, gn = ops.fc_soft_bwd(x, cand, w, npar, node_kind, inv_tau, gy, need_x, need_conn,
+                                 need_raw)
+    gconn, (graw,) = ops.layer_params_bwd(w, gw, [raw], node_kind, 2, 1.0, gn, need_conn, [need_raw])
+    return tuple(g if g is not None else _empty(x) for g in (gx, gconn, graw))
+
+
+@fc_layer_bwd.register_fake
+def _(x, cand, raw, w, npar, node_kind, inv_tau, gy, need_x, need_conn, need_raw):
+    return tuple(x.new_empty(t.shape if n else (0,), dtype=torch.float32)
+                 for t, n in ((x, need_x), (w, need_conn), (raw, need_raw)))
+
+
+def _fc_layer_setup(ctx, inputs, output):
+    x, cand, conn, raw, node_kind, inv_tau = inputs
+    ctx.mark_non_differentiable(output[1], output[2])
+    ctx.set_materialize_grads(False)   # no zero tensors in their place
+    ctx.save_for_backward(x, cand, raw, output[1], output[2])
+    ctx.meta = (node_kind, inv_tau)
+
+
+def _fc_layer_backward(ctx, gy, _gw, _gn):
+    x, cand, raw, w, npar = ctx.saved_tensors
+    need = ctx.needs_input_grad
+    gx, gc, gr = fc_layer_bwd(x, cand, raw, w, npar, *ctx.meta, gy, need[0], need[2], need[3])
+    return _none(gx, need[0]), None, _none(gc, need[2]), _none(gr, need[3]), None, None
+
+
+fc_layer.register_autograd(_fc_layer_backward, setup_context=_fc_layer_setup)
+
+
+@torch.library.custom_op(f"{_NS}::fc_lut_layer", mutates_args=())
+def fc_lut_layer(x: Tensor, cand: Tensor, conn: Optional[Tensor], logits: Tensor,
+                 hybrid: bool) -> Tuple[Tensor, Tensor, Tensor]:
+    """LUT layer: ``cand/conn [OUT,n,K]``, ``logits [OUT,2^n]`` ->
+    ``(y [B,OUT], w, s)``."""
+    ops.require_gpu(x, cand, conn, logits)
+    cand = ops._c(cand, torch.int32)
+    w, s = ops.layer_params(conn, tuple(cand.shape), [logits], ops.HYBRID, cand.shape[1])
+    s = s.view(logits.shape)
+    return ops._fc_lut_launch(ops._as_f32(x), cand, w, s, hybrid), w, s
+
+
+@fc_lut_layer.register_fake
+def _(x, cand, conn, logits, hybrid):
+    return _layer_outputs(x, (x.shape[0], cand.shape[0]), cand.shape, logits.shape)
+
+
+@torch.library.custom_op(f"{_NS}::fc_lut_layer_bwd", mutates_args=())
+def fc_lut_layer_bwd(x: Tensor, cand: Tensor, logits: Tensor, w: Tensor, s: Tensor, gy: Tensor,
+                     need_x: bool, need_conn: bool,
+                     need_logits: bool) -> Tuple[Tensor, Tensor, Tensor]:
+    """``(gx, gconn, glogits)`` of fc_lut_layer; unneeded ones are empty."""
+    got = ops.fc_lut_soft_bwd(x, cand, w, s, gy, need_x, need_conn, need_logits)
+    if got is None:
+        raise NotImplementedError("fc_lut_layer backward: the input width exceeds what the "
+                                  "kernels stage in LDS")
+    gx, gw, gs = got
+    gconn, (gl,) = ops.layer_params_bwd(w, gw, [logits], ops.HYBRID, cand.shape[1], 1.0, gs,
+                                        need_conn, [need_logits])
+    return tuple(g if g is not None else _empty(x) for g in (gx, gconn, gl))
+
+
+@fc_lut_layer_bwd.register_fake
+def _(x, cand, logits, w, s, gy, need_x, need_conn, need_logits):
+    return tuple(x.new_empty(t.shape if n else (0,), dtype=torch.float32)
+                 for t, n in ((x, need_x), (w, need_conn), (logits, need_logits)))
+
+
+def _fc_lut_layer_setup(ctx, inputs, output):
+    x, cand, conn, logits, hybrid = inputs
+    ctx.mark_non_differentiable(output[1], output[2])
+    ctx.set_materialize_grads(False)   # no zero tensors in their place
+    ctx.save_for_backward(x, cand, logits, output[1], output[2])
+
+
+def _fc_lut_layer_backward(ctx, gy, _gw, _gs):
+    x, cand, logits, w, s = ctx.saved_tensors
+    need = ctx.needs_input_grad
+    gx, gc, gl = fc_lut_layer_bwd(x, cand, logits, w, s, gy, need[0], need[2], need[3])
+    return _none(gx, need[0]), None, _none(gc, need[2]), _none(gl, need[3]), None
+
+
+fc_lut_layer.register_autograd(_fc_lut_layer_backward, setup_context=_fc_lut_layer_setup)
+
+
+# ---------------------------------------------------------------------------
 # LUT FC layer (multilinear_logic)
 # ---------------------------------------------------------------------------
 @torch.library.custom_op(f"{_NS}::fc_lut_soft", mutates_args=())
@@ -324,6 +441,92 @@ def _conv_backward(ctx, gy):
 
 
 conv_soft.register_autograd(_conv_backward, setup_context=_conv_setup)
+
+
+def _levels(*ls):
+    return [t for t in ls if t is not None]
+
+
+@torch.library.custom_op(f"{_NS}::conv_layer", mutates_args=())
+def conv_layer(x: Tensor, conn: Optional[Tensor], l0: Tensor, l1: Optional[Tensor],
+               l2: Optional[Tensor], l3: Optional[Tensor], l4: Optional[Tensor],
+               basis: Optional[Tensor], cm: Tensor, ch: Tensor, cw: Tensor, node_kind: int,
+               depth: int, arity: int, K: int, pad: int, pool: bool,
+               scale: float) -> Tuple[Tensor, Tensor, Tensor]:
+    """Conv tree block from its own parameters (``conn [N,leaves,K]`` and one
+    raw tensor per tree level, gate16: the ``basis [16,4]``) -> ``(y, w
+    [N,leaves,K], npar [N,nodes,P])``."""
+    ops.require_gpu(x, conn, l0, cm)
+    cm, ch, cw = (ops._c(t, torch.int32) for t in (cm, ch, cw))
+    levels = _levels(l0, l1, l2, l3, l4)
+    if node_kind == ops.GATE16:
+        # the coefficients by torch's product: its order of the 16 terms
+        # follows the row count, and one bit of a coefficient moves the pooled
+        # routing of every near-tie
+        w = (torch.ones(cm.shape, device=x.device) if conn is None else
+             torch.softmax(conn, 2))
+        npar = torch.softmax(torch.cat(levels, 1), 2) @ basis
+    else:
+        w, npar = ops.layer_params(conn, tuple(cm.shape), levels, node_kind,
+                                   2 if node_kind == ops.WALSH else arity, scale)
+    y = ops._conv_soft_launch(ops._as_f32(x), npar, w, cm, ch, cw, node_kind, depth, arity, K, pad,
+                              pool)
+    return y, w, npar
+
+
+@conv_layer.register_fake
+def _(x, conn, l0, l1, l2, l3, l4, basis, cm, ch, cw, node_kind, depth, arity, K, pad, pool,
+      scale):
+    _, nodes, P = ops.tree_shape(node_kind, depth, arity)
+    return _layer_outputs(x, _conv_out_shape(x, cm, pad, pool), cm.shape, (cm.shape[0], nodes, P))
+
+
+@torch.library.custom_op(f"{_NS}::conv_layer_bwd", mutates_args=())
+def conv_layer_bwd(x: Tensor, l0: Tensor, l1: Optional[Tensor], l2: Optional[Tensor],
+                   l3: Optional[Tensor], l4: Optional[Tensor], w: Tensor, npar: Tensor, cm: Tensor,
+                   ch: Tensor, cw: Tensor, node_kind: int, depth: int, arity: int, K: int,
+                   pad: int, pool: bool, scale: float, gy: Tensor, need_x: bool, need_conn: bool,
+                   need_levels: List[bool]
+                   ) -> Tuple[Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor]:
+    """``(gx, gconn, gl0 .. gl4)`` of conv_layer; unneeded ones are empty."""
+    levels = _levels(l0, l1, l2, l3, l4)
+    got = ops.conv_soft_bwd(x, npar, w, cm, ch, cw, node_kind, depth, arity, K, pad, pool, gy, need_x,
+                            any(need_levels), need_conn)
+    if got is None:
+        raise NotImplementedError("conv_layer backward: shape outside the HIP kernels")
+    gx, gn, gw = got
+    gconn, gl = ops.layer_params_bwd(w, gw, levels, node_kind,
+                                     2 if node_kind in (ops.GATE16, ops.WALSH) else arity, scale,
+                                     gn, need_conn, need_levels[:len(levels)])
+    gl = gl + [None] * (5 - len(gl))
+    return tuple(g if g is not None else _empty(x) for g in (gx, gconn, *gl))
+
+
+@conv_layer_bwd.register_fake
+def _(x, l0, l1, l2, l3, l4, w, npar, cm, ch, cw, node_kind, depth, arity, K, pad, pool, scale, gy,
+      need_x, need_conn, need_levels):
+    need = [need_x, need_conn] + list(need_levels)
+    return tuple(x.new_empty(t.shape if n and t is not None else (0,), dtype=torch.float32)
+                 for t, n in zip((x, w, l0, l1, l2, l3, l4), need))
+
+
+def _conv_layer_setup(ctx, inputs, output):
+    x, conn, l0, l1, l2, l3, l4, basis, cm, ch, cw = inputs[:11]
+    ctx.mark_non_differentiable(output[1], output[2])
+    ctx.set_materialize_grads(False)   # no zero tensors in their place
+    ctx.save_for_backward(x, l0, l1, l2, l3, l4, output[1], output[2], cm, ch, cw)
+    ctx.meta = tuple(inputs[11:])
+
+
+def _conv_layer_backward(ctx, gy, _gw, _gn):
+    need = ctx.needs_input_grad
+    gx, gc, *gl = conv_layer_bwd(*ctx.saved_tensors, *ctx.meta, gy, need[0], need[1],
+                                 [bool(n) for n in need[2:7]])
+    return (_none(gx, need[0]), _none(gc, need[1]),
+            *(_none(g, n) for g, n in zip(gl, need[2:7]))) + (None,) * 11
+
+
+conv_layer.register_autograd(_conv_layer_backward, setup_context=_conv_layer_setup)
 
 
 # The reference's tree_conv / tree_conv_topk signature (kernels/conv.py:399-400,

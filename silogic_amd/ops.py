@@ -173,6 +173,68 @@ def fc_soft(x, cand, w, npar, node_kind, inv_tau=1.0):
 
 
 # ---------------------------------------------------------------------------
+# a training step's parameters
+# ---------------------------------------------------------------------------
+def param_levels_ok(conn, levels, K):
+    """Whether ``slg_layer_params`` takes a layer's parameters: plain fp32
+    tensors on the GPU, contiguous, aligned for 16-byte loads, at most 16
+    candidates and 5 tree levels. Calls under a ``torch.func`` transform keep
+    the parameters' torch expressions, which it sees through; ``torch.compile``
+    traces the same operators as eager mode runs."""
+    if not 0 < len(levels) <= 5 or K > 16:
+        return False
+    ts = list(levels) if conn is None else [conn, *levels]
+    if not all(t.dtype == torch.float32 and t.is_cuda and t.is_contiguous() for t in ts):
+        return False
+    if torch.compiler.is_compiling():
+        return True
+    return torch._C._functorch.peek_interpreter_stack() is None and all(
+        type(t) in (torch.Tensor, torch.nn.Parameter) and t.data_ptr() % 16 == 0 for t in ts)
+
+
+_ONE_NODE = (ctypes.c_int32 * 1)(1)
+
+
+def _level_args(levels, N, P_raw):
+    if len(levels) == 1 and levels[0].numel() == N * P_raw:   # an FC layer, a tree of one node
+        return _ONE_NODE, 1
+    nodes = [t.numel() // (N * P_raw) for t in levels]
+    if any(t.numel() != N * P_raw * m for t, m in zip(levels, nodes)):
+        raise ValueError("layer_params: level shapes %s for %d channels"
+                         % ([tuple(t.shape) for t in levels], N))
+    return (ctypes.c_int32 * len(nodes))(*nodes), sum(nodes)
+
+
+def layer_params(conn, w_shape, levels, kind, arity, scale=1.0):
+    """``(w, npar)`` of a layer from its parameters in one launch: ``w``
+    (shape ``[N, ..., K]``) = softmax of ``conn`` (ones for None), ``npar``
+    ``[N, nodes, P]`` from the raw parameters of every tree level."""
+    N, K = w_shape[0], w_shape[-1]
+    P = 4 if kind in (GATE16, WALSH) else 2 ** arity
+    nodes, NN = _level_args(levels, N, 16 if kind == GATE16 else P)
+    dev = levels[0].device
+    w = torch.empty(w_shape, device=dev, dtype=torch.float32)
+    npar = torch.empty((N, NN, P), device=dev, dtype=torch.float32)
+    _lib.call("slg_layer_params", _p(conn), w.numel() // K, K, len(levels), _ptrs(levels), nodes, N,
+              kind, arity, float(scale), _p(w), _p(npar), _stream(levels[0]))
+    return w, npar
+
+
+def layer_params_bwd(w, gw, levels, kind, arity, scale, gnp, need_conn, need_levels):
+    """``(gconn, [level gradients])`` from the gradients of ``w`` and ``npar``
+    (None where not needed)."""
+    N, K = w.shape[0], w.shape[-1]
+    P = 4 if kind in (GATE16, WALSH) else 2 ** arity
+    nodes, _ = _level_args(levels, N, 16 if kind == GATE16 else P)
+    gconn = torch.empty_like(w) if need_conn else None
+    graw = [torch.empty_like(t) if n else None for t, n in zip(levels, need_levels)]
+    _lib.call("slg_layer_params_bwd", _p(w), _p(gw), w.numel() // K, K, len(levels), _ptrs(levels),
+              nodes, N, kind, arity, float(scale), _p(gnp), _p(gconn), _ptrs(graw),
+              _stream(levels[0]))
+    return gconn, graw
+
+
+# ---------------------------------------------------------------------------
 # FC layers of n-input LUT nodes (multilinear of any arity, hybrid)
 # ---------------------------------------------------------------------------
 def _fc_lut_launch(x, cand, w, s, hybrid):

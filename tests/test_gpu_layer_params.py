@@ -1,0 +1,93 @@
+"""The layers' training operators (``slg_layer_params`` and its backward inside
+``fc_layer``, ``fc_lut_layer``, ``conv_layer``) against the modules' torch
+expressions of the same parameters, every node kind, wiring and depth."""
+import pytest
+import torch
+
+import silogic_amd as sl
+from silogic_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+LAYERS = [("gate16", 2, "topk", 8, 1.0), ("gate16", 2, "fixed", 1, 1.0), ("gate16", 2, "topk", 16, 1.0),
+          ("walsh", 2, "topk", 5, 0.5), ("multilinear", 2, "blocktopk", 8, 1.0),
+          ("multilinear", 3, "topk", 4, 1.0), ("hybrid", 6, "topk", 8, 1.0),
+          ("hybrid", 2, "topk", 1, 1.0)]
+BLOCKS = [("gate16", 2, 1, "topk", 4, 1.0), ("gate16", 2, 2, "topk", 3, 1.0),
+          ("gate16", 2, 3, "fixed", 1, 1.0), ("gate16", 2, 4, "topk", 2, 1.0),
+          ("walsh", 2, 2, "topk", 4, 0.7), ("walsh", 2, 4, "topk", 2, 1.0),
+          ("multilinear", 6, 1, "topk", 8, 1.0), ("multilinear", 3, 2, "topk", 2, 1.0),
+          ("hybrid", 4, 1, "topk", 4, 1.0)]
+
+
+def _both(monkeypatch, module, x, call, used):
+    """Outputs and gradients on the operators and on the torch expressions."""
+    got = []
+    for on in (True, False):
+        if not on:
+            monkeypatch.setattr(ops, "param_levels_ok", lambda *a: False)
+        x.grad = None
+        module.zero_grad(set_to_none=True)
+        y = call(x)
+        assert (used in y.grad_fn.__class__.__name__ or used in str(y.grad_fn.name())) == on
+        gy = torch.randn(y.shape, generator=torch.Generator().manual_seed(1)).cuda()
+        y.backward(gy)
+        got.append([y.detach(), x.grad] + [p.grad for p in module.parameters()])
+    return got
+
+
+def _close(a, b):
+    for s, t in zip(a, b):
+        assert (s is None) == (t is None)
+        if s is not None:
+            # the two derive the parameters with a few fp32 roundings each
+            # (softmax of 16, a product over 16): 32 eps of the tensor's norm
+            assert (s - t).norm() <= 32 * 2.0 ** -23 * (t.norm() + 1e-6)
+
+
+@pytest.mark.parametrize("node,arity,wiring,k,tau", LAYERS)
+def test_fc_layers(monkeypatch, node, arity, wiring, k, tau):
+    torch.manual_seed(0)
+    m = sl.LogicLayer(37, 70, node=node, connectome=wiring, arity=arity, k=k, tau=tau, seed=1)
+    m = m.cuda().train()
+    with torch.no_grad():
+        for p in m.parameters():
+            p.copy_(torch.randn(p.shape))
+    x = torch.rand(9, 37).cuda().requires_grad_(True)
+    lut = m.is_lut
+    _close(*_both(monkeypatch, m, x, m, "fc_lut_layer" if lut else "fc_layer"))
+
+
+@pytest.mark.parametrize("node,arity,depth,wiring,k,tau", BLOCKS)
+def test_conv_blocks(monkeypatch, node, arity, depth, wiring, k, tau):
+    torch.manual_seed(0)
+    m = sl.ConvLogicTree(3, 5, tree_depth=depth, connect=wiring, k=k, node=node, arity=arity,
+                         tau=tau, residual_init=False, seed=2).cuda().train()
+    with torch.no_grad():
+        for p in m.parameters():
+            p.copy_(torch.randn(p.shape))
+    x = torch.rand(3, 3, 6, 8).cuda().requires_grad_(True)
+    _close(*_both(monkeypatch, m, x, m.forward_pooled, "conv_layer"))
+
+
+def test_frozen_parameters_and_input():
+    torch.manual_seed(0)
+    m = sl.LogicLayer(20, 30, k=4, seed=1).cuda().train()
+    m.node.gate_logits.requires_grad_(False)
+    x = torch.rand(5, 20).cuda()
+    g, = torch.autograd.grad(m(x).sum(), [m._conn.conn])
+    m.node.gate_logits.requires_grad_(True)
+    g2, gl = torch.autograd.grad(m(x).sum(), [m._conn.conn, m.node.gate_logits])
+    assert torch.equal(g, g2) and gl.shape == (30, 16)
+
+
+def test_other_dtypes_and_transforms_keep_their_path():
+    m = sl.LogicLayer(20, 30, k=4, seed=1).cuda().train()
+    assert ops.param_levels_ok(m._conn.conn, [m.node.gate_logits], 4)
+    assert not ops.param_levels_ok(m._conn.conn, [m.node.gate_logits.double()], 4)
+    assert not ops.param_levels_ok(m._conn.conn.transpose(0, 2), [m.node.gate_logits], 4)
+    assert not ops.param_levels_ok(None, [torch.empty(30 * 16 + 1).cuda()[1:].view(30, 16)], 4)
+    seen = []
+    torch.func.grad(lambda c: (seen.append(ops.param_levels_ok(c, [c], 4)), c.sum())[1])(
+        torch.ones(4).cuda())
+    assert seen == [False]
