@@ -72,16 +72,13 @@ __global__ void __launch_bounds__(256) ig_keys_kernel(IgArgs a, const int* __res
 // sum). perm [group][IB]: each slot's input | its count << 16, and the heavy
 // inputs from the end; slot [key] (heavy inputs: -1); off: the first entry of
 // each chunk of 64 slots.
-__global__ void __launch_bounds__(1024) ig_slots_kernel(IgArgs a, const int* __restrict__ start,
-                                                        int* __restrict__ perm,
-                                                        int* __restrict__ slot,
-                                                        int* __restrict__ off,
-                                                        int* __restrict__ heavy) {
+// s[0..IB]: where each input's references start; first: the group's first entry.
+__device__ inline void ig_group_slots(const IgArgs& a, int g, const int* s, int first,
+                                      int* __restrict__ perm, int* __restrict__ slot,
+                                      int* __restrict__ off, int* __restrict__ heavy) {
   __shared__ int hist[kHeavy + 2], at[kHeavy + 2], part[16];
-  const int g = blockIdx.x, q = g % a.NB;
-  const int n = min(a.IB, a.IN - q * a.IB);  // inputs of the block
+  const int n = min(a.IB, a.IN - g % a.NB * a.IB);  // inputs of the block
   const int t = threadIdx.x;
-  const int* s = start + (int64_t)g * a.IB;
   int* pm = perm + (int64_t)g * a.IB;
   int* sl = slot + (int64_t)g * a.IB;
   for (int i = t; i < kHeavy + 2; i += 1024) hist[i] = 0;
@@ -130,9 +127,18 @@ __global__ void __launch_bounds__(1024) ig_slots_kernel(IgArgs a, const int* __r
   }
   if (lane == 63) part[wave] = x;
   __syncthreads();
-  int base = s[0] + g * ig_slack(a.IB);
+  int base = first + g * ig_slack(a.IB);
   for (int w = 0; w < wave; ++w) base += part[w];
   if (t < kIgWaves * kIgSlots && c < NC) off[(int64_t)g * NC + c] = base + x - len;
+}
+
+__global__ void __launch_bounds__(1024) ig_slots_kernel(IgArgs a, const int* __restrict__ start,
+                                                        int* __restrict__ perm,
+                                                        int* __restrict__ slot,
+                                                        int* __restrict__ off,
+                                                        int* __restrict__ heavy) {
+  const int* s = start + (int64_t)blockIdx.x * a.IB;
+  ig_group_slots(a, blockIdx.x, s, s[0], perm, slot, off, heavy);
 }
 
 // Entries (LDS byte offset of the row within its pass, weight) of each
@@ -158,6 +164,98 @@ __global__ void __launch_bounds__(256) ig_entries_kernel(IgArgs a, const int* __
     const int NC = (a.IB + 63) >> 6;
     const int64_t at = off[(int64_t)(key / a.IB) * NC + (s >> 6)] + (int64_t)(j - start[key]) * 64 + (s & 63);
     ent[at] = e;
+  }
+}
+
+// The whole table in one launch, a workgroup per input block, for one pass
+// (ig_small): the references that fall in the block are counted, placed and
+// ranked in LDS, where the eight launches of the general way pass everything
+// through memory. Each workgroup reads all candidates, twice.
+__global__ void __launch_bounds__(1024)
+ig_table_kernel(IgArgs a, const int* __restrict__ cand, const float* __restrict__ w,
+                int* __restrict__ start, int* __restrict__ perm, int* __restrict__ slot,
+                int* __restrict__ off, int* __restrict__ heavy, int2* __restrict__ ent,
+                int2* __restrict__ ent_heavy) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  __shared__ int part[16], before[16];
+  int* cur = reinterpret_cast<int*>(smem);                              // [IB + 1]
+  uint16_t* refs = reinterpret_cast<uint16_t*>(cur + a.IB + 1);         // [R]
+  const int g = blockIdx.x, i0 = g * a.IB, R = (int)a.R;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  for (int i = t; i <= a.IB; i += 1024) cur[i] = 0;
+  __syncthreads();
+  auto input = [&](int r) { return min(max(cand[r], 0), a.IN - 1) - i0; };  // within the block
+  auto each = [&](auto&& f) {  // f(r, input) over the references, 16 loads in flight
+    constexpr int U = 16;
+    for (int r0 = t; r0 < R; r0 += U * 1024) {
+      int i[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) i[u] = cand[min(r0 + u * 1024, R - 1)];
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (r0 + u * 1024 < R) f(r0 + u * 1024, min(max(i[u], 0), a.IN - 1) - i0);
+    }
+  };
+  int low = 0;  // references of earlier blocks
+  each([&](int, int i) {
+    low += i < 0;
+    if ((unsigned)i < (unsigned)a.IB) atomicAdd(&cur[i], 1);
+  });
+  __syncthreads();
+  // exclusive scan of the counts, a run of them per thread
+  const int per = (a.IB + 1023) / 1024, c0 = min(t * per, a.IB), c1 = min(c0 + per, a.IB);
+  int sum = 0;
+  for (int i = c0; i < c1; ++i) sum += cur[i];
+  int x = sum;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int y = __shfl_up(x, d, 64);
+    if (lane >= d) x += y;
+    low += __shfl_xor(low, d, 64);
+  }
+  if (lane == 63) part[wave] = x;
+  if (lane == 0) before[wave] = low;
+  __syncthreads();
+  int at = x - sum, first = 0, all = 0;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) {
+    at += v < wave ? part[v] : 0;
+    all += part[v];
+    first += before[v];
+  }
+  for (int i = c0; i < c1; ++i) {
+    const int c = cur[i];
+    cur[i] = at;
+    start[i0 + i] = first + at;
+    at += c;
+  }
+  if (t == 0) {
+    cur[a.IB] = all;
+    if (g == a.NB - 1) start[i0 + a.IB] = first + all;
+  }
+  __syncthreads();
+  ig_group_slots(a, g, cur, first, perm, slot, off, heavy);
+  __threadfence_block();
+  __syncthreads();
+  // place: afterwards cur[i] is the end of input i's list, cur[i - 1] its start
+  each([&](int r, int i) {
+    if ((unsigned)i < (unsigned)a.IB) refs[atomicAdd(&cur[i], 1)] = (uint16_t)r;
+  });
+  __syncthreads();
+  const int SK = a.NS * a.K, NC = (a.IB + 63) >> 6;
+  for (int j = t; j < all; j += 1024) {
+    const int r = refs[j], i = input(r);
+    const int b = i ? cur[i - 1] : 0, e = cur[i];
+    int rank = 0;  // ascending references, whatever order they were placed in
+    for (int k = b; k < e; ++k) rank += refs[k] < r;
+    const int o = r / SK, side = (r - o * SK) / a.K;
+    const int2 v = make_int2((side * a.OUT + o) * 16, __float_as_int(w[r]));
+    const int sl = slot[i0 + i];
+    if (sl < 0)
+      ent_heavy[first + b + rank] = v;
+    else
+      ent[(int64_t)off[(int64_t)g * NC + (sl >> 6)] + (int64_t)rank * 64 + (sl & 63)] = v;
   }
 }
 
@@ -370,6 +468,22 @@ int64_t fc_input_grad_floats(int64_t B, int64_t IN, int64_t OUT, int nsides, int
   return ig_plan(B, IN, OUT, nsides, K).total;
 }
 
+// One launch for the whole table: one pass, lists of 32 references on average
+// at most (an element's rank reads its list) and at most 4096 references a
+// block, 48K in all: a workgroup's scattered loads and stores bound it, so it
+// follows the references of a block, and every block reads all of them. FC
+// backward, K = 8, this against the general way, captured: 250 -> 250, B = 64:
+// 40 / 46 us; 1000, B = 256 (4000 a block): 57 / 63; 3000, B = 64 (4000 a
+// block, 48000 in all): 67 / 68; past the rule 4000, B = 64: 77 / 75; 2000,
+// B = 256 (8000 a block): 81 / 73; 1000, B = 1024 (16000): 98 / 76.
+static size_t ig_small_lds(const IgArgs& a) {
+  return (size_t)(a.IB + 1) * 4 + (size_t)a.R * 2;
+}
+static bool ig_small(const IgArgs& a) {
+  return a.NP == 1 && a.R <= 48 * 1024 && a.R <= 32 * (int64_t)a.IN && a.R <= 4096 * (int64_t)a.NB &&
+         ig_small_lds(a) <= 150 * 1024;
+}
+
 int fc_input_grad(const float* gbr, int64_t B, int64_t IN, int64_t OUT, int nsides, int K,
                   const int32_t* cand, const float* w, float* ws, float* gx, hipStream_t st) {
   const IgPlan p = ig_plan(B, IN, OUT, nsides, K);
@@ -383,15 +497,28 @@ int fc_input_grad(const float* gbr, int64_t B, int64_t IN, int64_t OUT, int nsid
       *heavy = iw + p.heavy;
   int2* ent = reinterpret_cast<int2*>(iw + p.ent);
   int2* ent_heavy = reinterpret_cast<int2*>(iw + p.ent_heavy);
-  const unsigned rb = (unsigned)cdiv(a.R, 256);
-  hipLaunchKernelGGL(ig_keys_kernel, dim3(rb), dim3(256), 0, st, a, cand, keys);
   RefTable tb{};
-  const int rc = build_ref_table(keys, a.R, p.nkeys, iw + p.table, st, &tb);
-  if (rc) return rc;
-  hipLaunchKernelGGL(ig_slots_kernel, dim3((unsigned)p.groups), dim3(1024), 0, st, a, tb.start, perm,
-                     slot, off, heavy);
-  hipLaunchKernelGGL(ig_entries_kernel, dim3(rb), dim3(256), 0, st, a, tb.sorted, keys, tb.start, slot,
-                     off, w, ent, ent_heavy);
+  if (ig_small(a)) {
+    tb.start = iw + p.table;
+    const size_t lds = ig_small_lds(a);
+    if (lds > 65536 - 8192) {
+      const hipError_t e = hipFuncSetAttribute((const void*)ig_table_kernel,
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+      SLG_REQUIRE(e == hipSuccess, (int)e, "fc input gradient: LDS %zu: %s", lds,
+                  hipGetErrorString(e));
+    }
+    hipLaunchKernelGGL(ig_table_kernel, dim3((unsigned)a.NB), dim3(1024), lds, st, a, cand, w, tb.start,
+                       perm, slot, off, heavy, ent, ent_heavy);
+  } else {
+    const unsigned rb = (unsigned)cdiv(a.R, 256);
+    hipLaunchKernelGGL(ig_keys_kernel, dim3(rb), dim3(256), 0, st, a, cand, keys);
+    const int rc = build_ref_table(keys, a.R, p.nkeys, iw + p.table, st, &tb);
+    if (rc) return rc;
+    hipLaunchKernelGGL(ig_slots_kernel, dim3((unsigned)p.groups), dim3(1024), 0, st, a, tb.start, perm,
+                       slot, off, heavy);
+    hipLaunchKernelGGL(ig_entries_kernel, dim3(rb), dim3(256), 0, st, a, tb.sorted, keys, tb.start,
+                       slot, off, w, ent, ent_heavy);
+  }
   SLG_LAUNCH_CHECK("fc input gradient table");
   const size_t lds = (size_t)std::max(a.RB + 1, a.IB) * 16;
   if (lds > 65536) {
