@@ -86,6 +86,7 @@ struct SmArgs {
   int PS, RPS;        // row splits of the map, rows per split
   int ncg;            // chunk groups: a job takes chunks cg, cg + ncg, ...
   int TH, nt;         // sm_gx: rows per strip, strips per image
+  int GS;             // sm_gx: parts of a channel's taps, a wave each
   int Cz;             // channels stored: C, and a zero one for candidates past K
   int RS;             // record words
   int64_t xs;         // floats per chunk of the sample-minor image
@@ -777,18 +778,24 @@ sm_grad_kernel(SmArgs a, const uint32_t* __restrict__ recs, const float* __restr
 // strip are not loaded (an offset past the buffer reads 0). U outputs divide
 // the map's rows into equal steps; where they do not, the last step starts
 // early; the outputs it repeats, and those routed to a row outside the strip,
-// add to a per-lane dump slot.
+// add to a per-lane dump slot. Few strips of long lists (few channels under
+// many trees) would leave the chip idle: the list is then split over GS waves,
+// part 0 into gx, the others into images that sm_gx_sum adds in order (11
+// channels under 216 depth-3 trees, 12x12, 5x5, B = 126: 132 waves, 685 us
+// unsplit).
 template <bool POOL, int U, int NR>
 __global__ void __launch_bounds__(64)
 sm_gx_kernel(SmArgs a, int NLEAF, const int* __restrict__ start, const SmRef* __restrict__ refs,
              const float* __restrict__ gl, const uint32_t* __restrict__ route,
-             float* __restrict__ gx) {
+             float* __restrict__ gx, float* __restrict__ parts) {
   extern __shared__ __align__(16) float tile[];
   constexpr int S = POOL ? 2 : 1;
   const unsigned lid = xcd_logical_id(blockIdx.x, gridDim.x);
   const unsigned cs = lid / (unsigned)a.C;
   const int c = (int)(lid - cs * (unsigned)a.C);
-  const int chunk = (int)(cs / (unsigned)a.nt), strip = (int)(cs - (unsigned)chunk * a.nt);
+  const unsigned cp = cs / (unsigned)a.nt;
+  const int strip = (int)(cs - cp * (unsigned)a.nt);
+  const int chunk = (int)(cp / (unsigned)a.GS), part = (int)(cp - (unsigned)chunk * a.GS);
   if (chunk >= a.nc) return;
   const int lane = threadIdx.x;
   const int r0 = strip * a.TH, rows = min(a.TH, a.H - r0);
@@ -801,7 +808,8 @@ sm_gx_kernel(SmArgs a, int NLEAF, const int* __restrict__ start, const SmRef* __
   // output py, window row q, tap row dh is S py + q + dh - pad
   const int py_lo = max(0, (r0 + a.pad - a.kernel + 1 - (S - 1) + S * 8) / S - 8);
   const int py_hi = min(a.Ho - 1, (r0 + rows - 1 + a.pad) / S);
-  const int j_begin = start[c], j_end = start[c + 1];
+  const int j_first = start[c], nj = start[c + 1] - j_first, per = (nj + a.GS - 1) / a.GS;
+  const int j_begin = j_first + min(part * per, nj), j_end = j_first + min((part + 1) * per, nj);
   const int leaf_bytes = a.P * 256, row_bytes = a.RW * 256;
   const auto gr = uniform_rsrc(gl + (int64_t)chunk * a.N * NLEAF * a.P * 64, a.N * NLEAF * leaf_bytes);
   const auto rr = uniform_rsrc(POOL ? (const void*)(route + (int64_t)chunk * a.N * a.Ho * a.RW * 64) : gl,
@@ -829,7 +837,7 @@ sm_gx_kernel(SmArgs a, int NLEAF, const int* __restrict__ start, const SmRef* __
     const bool any = j < j_end;
     const SmRef e = ref(any ? j : 0);
     r.j0 = j;
-    r.j1 = any ? e.next : j;
+    r.j1 = any ? min(e.next, j_end) : j;
     r.e = e;
     const int lo = (int)(e.d >> 8) & 15, hi = (int)(e.d >> 12) & 15;
     const int gbase = (e.tree * NLEAF + (int)(e.d >> 16)) * leaf_bytes + px * 256;
@@ -914,7 +922,7 @@ sm_gx_kernel(SmArgs a, int NLEAF, const int* __restrict__ start, const SmRef* __
   const int b0 = chunk * 64;
   const int px16 = lane & 15, quad = lane >> 4;
   const int64_t CHW = (int64_t)a.C * a.H * a.W;
-  float* dst = gx + ((int64_t)c * a.H + r0) * a.W;
+  float* dst = (part ? parts + (part - 1) * (a.B * CHW) : gx) + ((int64_t)c * a.H + r0) * a.W;
   const int n = rows * a.W;
   for (int i0 = 0; i0 < n; i0 += 16) {
     const int i = i0 + px16;
@@ -931,6 +939,16 @@ sm_gx_kernel(SmArgs a, int NLEAF, const int* __restrict__ start, const SmRef* __
       }
     }
   }
+}
+
+// gx[i] += the parts' images, in order.
+__global__ void __launch_bounds__(256) sm_gx_sum_kernel(const float* __restrict__ parts, int n_parts,
+                                                        int64_t n, float* __restrict__ gx) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) return;
+  float s = gx[i];
+  for (int p = 0; p < n_parts; ++p) s += parts[p * n + i];
+  gx[i] = s;
 }
 
 // gw[i] = sum over slots s of part_w[s][i], gnp likewise: a workgroup takes
@@ -1005,7 +1023,7 @@ struct SmPlan {
   int64_t slots;     // partial slots over all rounds
   int nleaf, nparam, rec_words;
   // workspace offsets (4-byte words, multiples of 64)
-  int64_t recs, start, refs, xT, gT, route, gl, pw, pn, total;
+  int64_t recs, start, refs, xT, gT, route, gl, pw, pn, parts, total;
 };
 
 static constexpr int64_t kSmRoundFloats = int64_t(64) << 20;  // leaf gradients of a round
@@ -1054,6 +1072,9 @@ static bool sm_plan(int64_t B, int64_t C, int64_t H, int64_t W, int64_t N, int n
   if (a.TH > 2 && C * a.nc * cdiv(H, a.TH) < kSmJobs / 2) a.TH = 2;
   a.TH = (int)std::min<int64_t>(a.TH, H);
   a.nt = (int)cdiv(H, a.TH);
+  // parts of the taps while waves are missing, of 32 taps at least on average
+  a.GS = (int)std::max<int64_t>(1, std::min<int64_t>({16, kSmJobs / 2 / (C * a.nc * a.nt),
+                                                      N * p.nleaf * K / (32 * C)}));
   const int64_t rounds = cdiv(p.nc_total, a.nc);
   p.slots = rounds * a.ncg * a.PS;
   int64_t o = 0;
@@ -1071,6 +1092,7 @@ static bool sm_plan(int64_t B, int64_t C, int64_t H, int64_t W, int64_t N, int n
   p.gl = take(a.nc * gl1);
   p.pw = take(p.slots * N * p.nleaf * K);
   p.pn = take(p.slots * N * p.nparam);
+  p.parts = take((a.GS - 1) * std::min<int64_t>(B, a.nc * int64_t(64)) * C * H * W);
   p.total = o;
   return true;
 }
@@ -1084,7 +1106,7 @@ int64_t conv_sm_bwd_workspace(int64_t B, int64_t C, int64_t H, int64_t W, int64_
 
 // sm_gx_kernel for rows in steps of u outputs.
 using SmGxKernel = void (*)(SmArgs, int, const int*, const SmRef*, const float*, const uint32_t*,
-                            float*);
+                            float*, float*);
 template <bool POOL, int NR>
 static SmGxKernel sm_gx_rows(int u) {
   static const SmGxKernel k[8] = {sm_gx_kernel<POOL, 1, NR>, sm_gx_kernel<POOL, 2, NR>,
@@ -1166,10 +1188,16 @@ int conv_sm_bwd(const float* x, int64_t B, int64_t C, int64_t H, int64_t W, int6
                 (const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
             SLG_REQUIRE(e == hipSuccess, (int)e, "conv_soft_bwd: LDS %zu: %s", lds, hipGetErrorString(e));
           }
-          const int64_t jobs = cdiv((int64_t)C * a.nc * a.nt, 8) * 8;
+          const int64_t jobs = cdiv((int64_t)C * a.nc * a.nt * a.GS, 8) * 8;
           hipLaunchKernelGGL(kern, dim3((unsigned)jobs), dim3(64), lds, st, a, NL, start, refs, gl,
-                             route, gx + b0 * C * H * W);
+                             route, gx + b0 * C * H * W, ws + p.parts);
           SLG_LAUNCH_CHECK("conv_soft_bwd input gradient");
+          if (a.GS > 1) {
+            const int64_t n = (int64_t)a.B * C * H * W;
+            hipLaunchKernelGGL(sm_gx_sum_kernel, dim3((unsigned)cdiv(n, 256)), dim3(256), 0, st,
+                               ws + p.parts, a.GS - 1, n, gx + b0 * C * H * W);
+            SLG_LAUNCH_CHECK("conv_soft_bwd input gradient parts");
+          }
         }
       }
       return 0;

@@ -105,3 +105,12 @@ def test_conv_backward_matches_float64(case):
     _, gn, gw = ops.conv_soft_bwd(x, npar, w, cm, ch, cw, kind, depth, arity, K, kernel // 2, pool,
                                   gy, need_x=False)
     assert torch.equal(gn, got[1]) and torch.equal(gw, got[2])
+
+
+@pytest.mark.parametrize("case", [
+    ("gate16", 3, 2, 4, 2, 8, 8, 96, 5, 2, 65, True),       # lists in 16 parts, cut inside a leaf's taps
+    ("multilinear", 1, 6, 4, 1, 6, 37, 40, 3, 1, 3, False),  # one channel
+    ("walsh", 2, 2, 8, 3, 16, 16, 33, 3, 1, 130, True),     # a last chunk of two samples
+], ids=lambda c: c[0])
+def test_split_input_gradient_matches_float64(case):
+    test_conv_backward_matches_float64(case)
