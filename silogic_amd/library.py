@@ -466,6 +466,8 @@ def conv_layer(x: Tensor, conn: Optional[Tensor], l0: Tensor, l1: Optional[Tenso
         w = (torch.ones(cm.shape, device=x.device) if conn is None else
              torch.softmax(conn, 2))
         npar = torch.softmax(torch.cat(levels, 1), 2) @ basis
+        # autocast runs the product in 16 bits, a default dtype makes the ones
+        w, npar = ops._c(w, torch.float32), ops._c(npar, torch.float32)
     else:
         w, npar = ops.layer_params(conn, tuple(cm.shape), levels, node_kind,
                                    2 if node_kind == ops.WALSH else arity, scale)

@@ -70,6 +70,34 @@ def test_conv_blocks(monkeypatch, node, arity, depth, wiring, k, tau):
     _close(*_both(monkeypatch, m, x, m.forward_pooled, "conv_layer"))
 
 
+def test_conv_block_under_autocast_and_a_default_dtype(monkeypatch):
+    # the kernels read 32-bit parameters: autocast's 16-bit basis product and a
+    # 64-bit default's ones are converted first. The forward's parameters are
+    # the same values on both paths; the gate gradients pass a bf16 product on
+    # one side only: 2 roundings of 2^-8, of terms up to four times as large as
+    # what p (d - p.d) leaves of them
+    def both(wiring, k):
+        torch.manual_seed(0)
+        m = sl.ConvLogicTree(3, 5, connect=wiring, k=k, residual_init=False, seed=2).cuda().train()
+        x = torch.rand(3, 3, 6, 8).cuda().requires_grad_(True)
+        with monkeypatch.context() as mp:
+            return _both(mp, m, x, m.forward_pooled, "conv_layer")
+
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        got, want = both("topk", 4)
+    assert torch.equal(got[0], want[0])
+    for a, b in zip(got[1:], want[1:]):
+        assert (a - b).norm() <= 2.0 ** -5 * b.norm()
+    m = sl.ConvLogicTree(3, 5, connect="fixed", residual_init=False, seed=2).cuda().train()
+    x = torch.rand(3, 3, 6, 8).cuda()
+    want = m.forward_pooled(x)
+    torch.set_default_dtype(torch.float64)
+    try:
+        assert torch.equal(m.forward_pooled(x), want)
+    finally:
+        torch.set_default_dtype(torch.float32)
+
+
 def test_frozen_parameters_and_input():
     torch.manual_seed(0)
     m = sl.LogicLayer(20, 30, k=4, seed=1).cuda().train()
