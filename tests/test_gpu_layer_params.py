@@ -119,3 +119,20 @@ def test_other_dtypes_and_transforms_keep_their_path():
     torch.func.grad(lambda c: (seen.append(ops.param_levels_ok(c, [c], 4)), c.sum())[1])(
         torch.ones(4).cuda())
     assert seen == [False]
+
+
+@pytest.mark.parametrize("node", ["gate16", "walsh"])
+def test_operator_takes_parameters_at_any_offset(node):
+    # a traced layer calls the operator whatever its parameters' addresses
+    m = sl.LogicLayer(20, 30, node=node, k=4, seed=1).cuda().train()
+    x = torch.rand(5, 20).cuda()
+    got = []
+    for off in (0, 1):
+        raw = m.node.raw().detach()
+        flat = torch.empty(raw.numel() + off, device="cuda")
+        shifted = flat[off:].view(raw.shape).copy_(raw).requires_grad_(True)
+        assert (shifted.data_ptr() % 16 == 0) == (off == 0)
+        y = torch.ops.silogic_hip.fc_layer(x, m._conn.candidates_i32(), m._conn.conn, shifted,
+                                           m.node.kind, 1.0)[0]
+        got.append((y.detach(), torch.autograd.grad(y.sum(), shifted)[0]))
+    assert all(torch.equal(a, b) for a, b in zip(*got))
