@@ -380,26 +380,16 @@ __global__ void __launch_bounds__(256) fc_lut_bwd_c_kernel(const float* __restri
   for (int c2 = 0; c2 < NC2; ++c2) base[(int64_t)(c1 + (c2 << H1)) * OUT] = acc[c2];
 }
 
-// out = sum over ranges of part [NR][NC][OUT] in fixed order (16 columns per
-// workgroup, 16 thread rows over the ranges), scattered as
+// out = sum over ranges of part [NR][NC][OUT] in fixed order, scattered as
 //   weights (mode 0): column (slot j*KM + k, o) -> gw[(o*NA + j)*K + k] for k < K
 //   corners (mode 1): column (p, o) -> gs[o*NC + p].
-__global__ void __launch_bounds__(256) fc_lut_bwd_reduce_kernel(const float* __restrict__ part,
-                                                                int NR, int NC, int OUT, int mode,
-                                                                int NA, int KM, int K,
-                                                                float* __restrict__ out) {
-  __shared__ float rs[16][17];
-  const int col = threadIdx.x & 15, rw = threadIdx.x >> 4;
-  const int64_t t = (int64_t)blockIdx.x * 16 + col;
+__global__ void __launch_bounds__(kSumThreads)
+fc_lut_bwd_reduce_kernel(const float* __restrict__ part, int NR, int NC, int OUT, int mode, int NA,
+                         int KM, int K, float* __restrict__ out) {
+  const int64_t t = (int64_t)blockIdx.x * kSumCols + (threadIdx.x & 63);
   const int64_t n = (int64_t)NC * OUT;
-  float s = 0.0f;
-  if (t < n)
-    for (int r = rw; r < NR; r += 16) s += part[(int64_t)r * n + t];
-  rs[rw][col] = s;
-  __syncthreads();
-  if (rw != 0 || t >= n) return;
-  float sum = 0.0f;
-  for (int q = 0; q < 16; ++q) sum += rs[q][col];
+  const float sum = range_sum(part, NR, n, t);
+  if (threadIdx.x >= kSumCols || t >= n) return;
   const int c = (int)(t / OUT), o = (int)(t - (int64_t)c * OUT);
   if (mode == 0) {
     const int j = c / KM, k = c - j * KM;
@@ -742,13 +732,13 @@ int slg_fc_lut_soft_bwd(const float* x, int64_t B, int64_t IN, int64_t OUT, int3
   const int NRw = B > 0 ? p.NRw : 0, NRc = B > 0 ? p.NRc : 0;  // no samples: zeros
   if (gw) {
     const int NK = arity * p.KM;
-    hipLaunchKernelGGL(fc_lut_bwd_reduce_kernel, dim3((unsigned)cdiv((int64_t)NK * OUT, 16)),
-                       dim3(256), 0, st, partw, NRw, NK, (int)OUT, 0, arity, p.KM, K, gw);
+    hipLaunchKernelGGL(fc_lut_bwd_reduce_kernel, dim3((unsigned)cdiv((int64_t)NK * OUT, kSumCols)),
+                       dim3(kSumThreads), 0, st, partw, NRw, NK, (int)OUT, 0, arity, p.KM, K, gw);
   }
   if (gs) {
     const int NP = 1 << arity;
-    hipLaunchKernelGGL(fc_lut_bwd_reduce_kernel, dim3((unsigned)cdiv((int64_t)NP * OUT, 16)),
-                       dim3(256), 0, st, partc, NRc, NP, (int)OUT, 1, arity, p.KM, K, gs);
+    hipLaunchKernelGGL(fc_lut_bwd_reduce_kernel, dim3((unsigned)cdiv((int64_t)NP * OUT, kSumCols)),
+                       dim3(kSumThreads), 0, st, partc, NRc, NP, (int)OUT, 1, arity, p.KM, K, gs);
   }
   SLG_LAUNCH_CHECK("fc_lut_bwd_reduce");
   return 0;

@@ -1,4 +1,4 @@
-"""FC backward (``csrc/fc_bwd_input.hip``, ``csrc/fc_soft_bwd.hip``) against
+"""FC backward (``csrc/fc_bwd_input.hip``, ``csrc/fc_soft_bwd.hip``, ``csrc/fc_lut.hip``) against
 float64 at the edges of its tiling: several blocks of inputs and passes of
 rows, inputs of more references than a lane's list, an input heavy in one
 pass only, widths off the vector loads, batches off the 2- and 4-sample
@@ -88,3 +88,26 @@ def test_fc_lut_input_gradient_matches_float64(arity, IN, OUT, K, B):
     refs = OUT * arity * K / IN
     rel = ((gx.double() - want).norm() / want.norm()).item()
     assert rel < EPS * (refs ** 0.5 + 3 * arity + K), rel
+
+
+@pytest.mark.parametrize("arity,OUT,K,B", [(2, 1, 1, 1), (3, 65, 4, 9), (4, 63, 8, 700), (6, 70, 5, 1300)])
+def test_fc_lut_parameter_gradients_match_float64(arity, OUT, K, B):
+    # partial sums over one range of samples, a few, more than a step of 64
+    from silogic_amd import ops
+    IN = 40
+    gen = torch.Generator().manual_seed(5)
+    cand = torch.randint(0, IN, (OUT, arity, K), generator=gen).int().cuda()
+    w = torch.softmax(torch.randn(OUT, arity, K, generator=gen), 2).cuda()
+    s = torch.rand(OUT, 2 ** arity, generator=gen).cuda()
+    x, gy = torch.rand(B, IN, generator=gen).cuda(), torch.randn(B, OUT, generator=gen).cuda()
+    _, gw, gs = ops.fc_lut_soft_bwd(x, cand, w, s, gy, False, True, True)
+    w64, s64 = w.double().requires_grad_(True), s.double().requires_grad_(True)
+    v = (x.double()[:, cand.long().reshape(-1)].view(B, OUT, arity, K) * w64).sum(3)
+    t = s64.expand(B, OUT, -1)
+    for j in range(arity):
+        t = t[..., 0::2] + v[..., j:j + 1] * (t[..., 1::2] - t[..., 0::2])
+    want = torch.autograd.grad(t[..., 0], (w64, s64), gy.double())
+    # B terms of mixed sign, each after about 3 arity + K roundings
+    for got, ref in ((gw, want[0]), (gs, want[1])):
+        rel = ((got.double() - ref).norm() / ref.norm()).item()
+        assert rel < EPS * (B ** 0.5 + 3 * arity + K), rel
