@@ -18,19 +18,26 @@ __global__ void __launch_bounds__(256) ref_count_kernel(const int* __restrict__ 
 
 // One workgroup: start[0..n] = exclusive scan of cnt, cursor = start, 4096
 // counts a step (coalesced: 20000 counts took 13 us with a run of counts per
-// thread). cnt and cursor may be the same array: each element is read before
+// thread), a thread's four as one 16-byte access and one barrier a step: 20480
+// counts 14.8 us with single accesses and two barriers, 6.8 so. cnt and cursor may be the same array: each element is read before
 // it is written, by the one thread that owns it.
 __global__ void __launch_bounds__(1024) ref_scan_kernel(const int* cnt, int n,
                                                         int* __restrict__ start, int* cursor) {
-  __shared__ int part[16];
+  __shared__ int part[2][16];
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  int run = 0;
+  int run = 0, sums = 0;
+  // a thread's four counts as one access each way, where the arrays allow it
+  const bool quads =
+      (((uintptr_t)cnt | (uintptr_t)start | (uintptr_t)cursor) & 15) == 0;
   auto load = [&](int base, int (&c)[4]) {
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int i = base + 4 * t + u;
-      c[u] = i < n ? cnt[i] : 0;
+    const int i0 = base + 4 * t;
+    if (quads && i0 + 4 <= n) {
+      const int4 v = *reinterpret_cast<const int4*>(cnt + i0);
+      c[0] = v.x; c[1] = v.y; c[2] = v.z; c[3] = v.w;
+      return;
     }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) c[u] = i0 + u < n ? cnt[i0 + u] : 0;
   };
   int c[4], nx[4];
   load(0, nx);
@@ -45,26 +52,30 @@ __global__ void __launch_bounds__(1024) ref_scan_kernel(const int* cnt, int n,
       const int y = __shfl_up(x, d, 64);
       if (lane >= d) x += y;
     }
-    if (lane == 63) part[wave] = x;
+    if (lane == 63) part[sums][wave] = x;
     __syncthreads();
     int before = 0, all = 0;
 #pragma unroll
     for (int w = 0; w < 16; ++w) {
-      before += w < wave ? part[w] : 0;
-      all += part[w];
+      before += w < wave ? part[sums][w] : 0;
+      all += part[sums][w];
     }
-    int at = run + before + x - sum;
+    const int at = run + before + x - sum, i0 = base + 4 * t;
+    const int4 v = make_int4(at, at + c[0], at + c[0] + c[1], at + c[0] + c[1] + c[2]);
+    if (quads && i0 + 4 <= n) {
+      *reinterpret_cast<int4*>(start + i0) = v;
+      *reinterpret_cast<int4*>(cursor + i0) = v;
+    } else {
+      const int e[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int i = base + 4 * t + u;
-      if (i < n) {
-        start[i] = at;
-        cursor[i] = at;
-      }
-      at += c[u];
+      for (int u = 0; u < 4; ++u)
+        if (i0 + u < n) {
+          start[i0 + u] = e[u];
+          cursor[i0 + u] = e[u];
+        }
     }
     run += all;
-    __syncthreads();
+    sums ^= 1;  // the next step's barrier separates a buffer's reads from its next writes
   }
   if (t == 0) start[n] = run;
 }
