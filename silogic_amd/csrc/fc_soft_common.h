@@ -258,7 +258,10 @@ __device__ inline float range_sum(const float* __restrict__ part, int NR, int64_
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   float s0 = 0.0f, s1 = 0.0f;
   if (t < n) {
-    for (int r = wave; r < NR; r += 64) {
+    if (NR <= 16) {  // a range a row: the clamped loads would be mostly repeats
+      s0 = wave < NR ? part[(int64_t)wave * n + t] : 0.0f;
+      s1 = wave + 8 < NR ? part[(int64_t)(wave + 8) * n + t] : 0.0f;
+    } else for (int r = wave; r < NR; r += 64) {
       float a[4], b[4];
 #pragma unroll
       for (int u = 0; u < 4; ++u) {

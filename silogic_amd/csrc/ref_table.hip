@@ -19,8 +19,9 @@ __global__ void __launch_bounds__(256) ref_count_kernel(const int* __restrict__ 
 // One workgroup: start[0..n] = exclusive scan of cnt, cursor = start, 4096
 // counts a step (coalesced: 20000 counts took 13 us with a run of counts per
 // thread), a thread's four as one 16-byte access and one barrier a step: 20480
-// counts 14.8 us with single accesses and two barriers, 6.8 so. cnt and cursor may be the same array: each element is read before
-// it is written, by the one thread that owns it.
+// counts 14.8 us with single accesses and two barriers, 6.8 so. cnt and cursor
+// may be the same array: each element is read before it is written, by the one
+// thread that owns it.
 __global__ void __launch_bounds__(1024) ref_scan_kernel(const int* cnt, int n,
                                                         int* __restrict__ start, int* cursor) {
   __shared__ int part[2][16];
