@@ -1702,6 +1702,20 @@ static int node_leaves(int node, int depth, int arity) {
   return -1;
 }
 
+// The rule of conv_soft_dispatch: the layout picked for the sizes fits LDS.
+bool conv_forward_on_lds(int64_t C, int64_t H, int64_t W, int64_t N, int node, int depth, int arity,
+                         int K, int pad, bool pool) {
+  const int nleaf = node_leaves(node, depth, arity);
+  if (nleaf <= 0 || K < 1 || K > kMaxK) return false;
+  const int64_t Ho = pool ? H / 2 : H, Wo = pool ? W / 2 : W;
+  const int km = K <= 4 ? 4 : kMaxK, kernel = 2 * pad + 1;
+  const int lay = conv_pooled_layout(pool, node, nleaf, km, C, H, W, Ho, Wo, kernel, N);
+  if (lay != kLayoutPlain) return true;
+  const ConvGeom g = conv_geom(C, H, W, pad, pool, conv_phase_layout(pool, nleaf, km), Ho, Wo);
+  const int64_t cap = std::min<int64_t>(device_lds_bytes(), 160 * 1024);
+  return (int64_t)g.SST * 4 + kConvExtra * 4 <= cap && C * H * W * 4 < (1LL << 31);
+}
+
 // Records of slg_conv_soft_records (ARR = false: from the connection logits
 // and raw node parameters) or slg_conv_soft_records_arrays (ARR = true: from
 // slg_conv_soft_fwd's separate arrays), for the layout the forward picks.

@@ -32,6 +32,7 @@
 #include <algorithm>
 #include <type_traits>
 
+#include "conv_tree.h"
 #include "ref_table.h"
 
 namespace slg {
@@ -61,42 +62,6 @@ struct GenLevels {
     }
   }
 };
-
-__device__ inline float gen_sigmoid(float z) { return 1.0f / (1.0f + expf(-z)); }
-
-// Value of one node with children c[0..A) and parameters p (uniform).
-template <int NODE, int A>
-__device__ inline float gen_node(const float* c, const float* __restrict__ p) {
-  if constexpr (NODE == SLG_NODE_GATE16 || NODE == SLG_NODE_WALSH) {
-    const float a = c[0], b = c[1];
-    const float z = p[0] + p[1] * a + p[2] * b + p[3] * (a * b);
-    if constexpr (NODE == SLG_NODE_WALSH) return gen_sigmoid(z);
-    return z;
-  } else if constexpr (NODE == SLG_NODE_HYBRID) {
-    int addr = 0;
-#pragma unroll
-    for (int j = 0; j < A; ++j) addr |= (c[j] >= 0.5f ? 1 : 0) << j;
-    return p[addr];
-  } else {
-    // the reference's product form (nodes.py:174-178): corner factors a_j or
-    // (1 - a_j) multiplied in leaf order, then sum_p w_p * s_p added in
-    // corner order, each operation rounded on its own (no contraction), so
-    // that values the reference computes as equal (near-ties of a flat tree
-    // at binary leaves) are equal here too: the pooled routing depends on it
-#pragma clang fp contract(off)
-    constexpr int PP = 1 << A;
-    float acc = 0.0f;
-#pragma unroll
-    for (int e = 0; e < PP; ++e) {
-      float w = (e & 1) ? c[0] : 1.0f - c[0];
-#pragma unroll
-      for (int j = 1; j < A; ++j) w = w * ((e >> j) & 1 ? c[j] : 1.0f - c[j]);
-      const float term = w * p[e];
-      acc = e == 0 ? term : acc + term;
-    }
-    return acc;
-  }
-}
 
 // Leaf values at output position (yy, xx) of sample b, channel n: the
 // softmax-weighted sum over K taps (zero padding outside the image).
@@ -272,7 +237,14 @@ __device__ inline void gen_node_bwd(const float* c, float y, const float* __rest
   }
 }
 
+// Trees whose forward may run on the kernels that stage images in LDS; LDSF:
+// this one's does, and the window positions are those of its evaluation.
 template <int NODE, int A, int D>
+constexpr bool gen_lds_form() {
+  return NODE == SLG_NODE_GATE16 ? D <= 4 : NODE == SLG_NODE_MULTILINEAR2 && D == 1;
+}
+
+template <int NODE, int A, int D, bool LDSF>
 __global__ void __launch_bounds__(256)
 conv_generic_bwd_kernel(const float* __restrict__ x, int C, int H, int W, int N, int K, int kernel,
                         int pad, int pool, int Hf, int Wf, int Ho, int Wo, int nblk, int b_base,
@@ -298,11 +270,27 @@ conv_generic_bwd_kernel(const float* __restrict__ x, int C, int H, int W, int N,
   int qs = 0;
   if (pool) {
     float best = -INFINITY;
+    float keep[LDSF ? T::NN * T::P : 1];
+    if constexpr (LDSF) {
+#pragma unroll
+      for (int i = 0; i < T::NN * T::P; ++i) keep[i] = par[i];
+      if constexpr (NODE == SLG_NODE_MULTILINEAR2) {
+        constexpr int LG = ConvNode<NODE, A>::LG;
+#pragma unroll
+        for (int g = 0; g < T::P >> LG; ++g)
+          lut_group_coeffs<LG>(*reinterpret_cast<float(*)[1 << LG]>(keep + (g << LG)));
+      }
+    }
     for (int q = 0; q < 4; ++q) {
       gen_leaves<T::NLEAF>(lv, xb, C, H, W, n, K, kernel, pad, 2 * oy + (q >> 1), 2 * ox + (q & 1),
                            w, cm, ch, cw);
-      gen_eval<NODE, A, D>(val, par);
-      const float v = val[NV - 1];
+      float v;
+      if constexpr (LDSF) {
+        v = conv_tree_eval<NODE, T::NLEAF>(lv, keep);
+      } else {
+        gen_eval<NODE, A, D>(val, par);
+        v = val[NV - 1];
+      }
       if (v > best || q == 0) {
         best = v;
         qs = q;
@@ -560,6 +548,7 @@ int conv_generic_bwd(const float* x, int64_t B, int64_t C, int64_t H, int64_t W,
                      const float* w, const int* cm, const int* ch, const int* cw, const float* gy,
                      float* gx, float* gw, float* gnp, float* ws, int64_t ws_floats,
                      hipStream_t st) {
+  const bool on_lds = pool && conv_forward_on_lds(C, H, W, N, node, depth, arity, K, pad, pool);
   const int A = (node == SLG_NODE_GATE16 || node == SLG_NODE_WALSH) ? 2 : arity;
   const int kernel = 2 * pad + 1;
   const int64_t Hf = H + 2 * pad - kernel + 1, Wf = W + 2 * pad - kernel + 1;
@@ -603,9 +592,12 @@ int conv_generic_bwd(const float* x, int64_t B, int64_t C, int64_t H, int64_t W,
     SLG_LAUNCH_CHECK("conv_soft_bwd (generic) zero");
     const int rc = gen_dispatch(node, A, depth, [&](auto nd, auto a_, auto d_) -> int {
       constexpr int NODE = decltype(nd)::value, AA = decltype(a_)::value, DD = decltype(d_)::value;
+      auto kern = conv_generic_bwd_kernel<NODE, AA, DD, false>;
+      if constexpr (gen_lds_form<NODE, AA, DD>()) {
+        if (on_lds) kern = conv_generic_bwd_kernel<NODE, AA, DD, true>;
+      }
       // part rows of this chunk start at slot b0 * nblk * 4
-      hipLaunchKernelGGL((conv_generic_bwd_kernel<NODE, AA, DD>),
-                         dim3((unsigned)(p.nblk * bc), (unsigned)N), dim3(256), 0, st, x, (int)C,
+      hipLaunchKernelGGL(kern, dim3((unsigned)(p.nblk * bc), (unsigned)N), dim3(256), 0, st, x, (int)C,
                          (int)H, (int)W, (int)N, K, kernel, pad, (int)pool, (int)Hf, (int)Wf, (int)Ho,
                          (int)Wo, (int)p.nblk, (int)b0, np, w, cm, ch, cw, gy,
                          part + b0 * p.nblk * 4 * p.R, p.slots, gleaf);

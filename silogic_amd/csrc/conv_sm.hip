@@ -89,6 +89,7 @@ struct SmArgs {
   int GS;             // sm_gx: parts of a channel's taps, a wave each
   int Cz;             // channels stored: C, and a zero one for candidates past K
   int RS;             // record words
+  int raw;            // the forward runs through the caches: the parameters kept as they are
   int64_t xs;         // floats per chunk of the sample-minor image
 };
 
@@ -207,15 +208,17 @@ sm_tables_kernel(SmArgs a, int rb, const float* __restrict__ np, const float* __
       float f = p[e];
       if constexpr (!T::kBinary) {
         const float mine = f;
-        if constexpr (NODE != SLG_NODE_HYBRID) {  // the forward's kept form (lut_group_coeffs)
-          constexpr int LG = ConvNode<NODE, NLEAF>::LG, GM = (1 << LG) - 1;
-          float g[1 << LG];
+        if constexpr (NODE != SLG_NODE_HYBRID) {  // the form of the forward on LDS (lut_group_coeffs)
+          if (!a.raw) {
+            constexpr int LG = ConvNode<NODE, NLEAF>::LG, GM = (1 << LG) - 1;
+            float g[1 << LG];
 #pragma unroll
-          for (int u = 0; u <= GM; ++u) g[u] = p[(e & ~GM) + u];
-          lut_group_coeffs<LG>(g);
-          f = g[0];
+            for (int u = 0; u <= GM; ++u) g[u] = p[(e & ~GM) + u];
+            lut_group_coeffs<LG>(g);
+            f = g[0];
 #pragma unroll
-          for (int u = 1; u <= GM; ++u) f = (e & GM) == u ? g[u] : f;
+            for (int u = 1; u <= GM; ++u) f = (e & GM) == u ? g[u] : f;
+          }
         }
         rec[R::pair + e] = __float_as_uint((e & 1) ? mine - p[e - 1] : mine);
       }
@@ -310,16 +313,13 @@ __device__ inline SmWords sm_words(const uint32_t* p) {
   return (SmWords)a;
 }
 
-__device__ inline float sm_sigmoid(float z) { return 1.0f / (1.0f + expf(-z)); }
-
-// c0 + c1 a + c2 b + c3 ab, the forward's three FMAs.
-__device__ inline float sm_bilinear(float a, float b, const float* c) {
-  return fmaf(b, fmaf(a, c[3], c[2]), fmaf(a, c[1], c[0]));
-}
-
-template <int NODE, int NLEAF>
+// The tree's value as the forward computes it: on the kernels that stage
+// images in LDS (LDS), or through the caches, node by node. par: the record's.
+template <int NODE, int NLEAF, bool LDS>
 __device__ inline float sm_eval(const float (&v)[NLEAF], const float* par) {
-  if constexpr (NODE == SLG_NODE_WALSH) {
+  if constexpr (LDS) {
+    return conv_tree_eval<NODE, NLEAF>(v, par);
+  } else if constexpr (SmTree<NODE, NLEAF>::kBinary) {
     float u[NLEAF];
 #pragma unroll
     for (int l = 0; l < NLEAF; ++l) u[l] = v[l];
@@ -327,15 +327,18 @@ __device__ inline float sm_eval(const float (&v)[NLEAF], const float* par) {
 #pragma unroll
     for (int cnt = NLEAF; cnt > 1; cnt >>= 1) {
 #pragma unroll
-      for (int m = 0; m < cnt / 2; ++m)
-        u[m] = sm_sigmoid(sm_bilinear(u[2 * m], u[2 * m + 1], par + 4 * (nb + m)));
+      for (int m = 0; m < cnt / 2; ++m) u[m] = gen_node<NODE, 2>(u + 2 * m, par + 4 * (nb + m));
       nb += cnt / 2;
     }
     return u[0];
   } else {
-    return conv_tree_eval<NODE, NLEAF>(v, par);
+    return gen_node<NODE, NLEAF>(v, par);
   }
 }
+
+// Walsh trees have no LDS forward.
+template <int NODE>
+constexpr bool sm_lds_form() { return NODE != SLG_NODE_WALSH; }
 
 // Leaf gradients of a binary tree (node ids level-major) at leaf values v
 // for upstream gradient g; each node's parameter gradient U * (1, a, b, ab)
@@ -349,9 +352,13 @@ __device__ inline void sm_grad_binary(const float (&v)[NLEAF], const float* par,
   for (int l = 0; l < NLEAF; ++l) val[l] = v[l];
 #pragma unroll
   for (int i = 0; i < NN; ++i) {  // node i's children are values 2i, 2i + 1
-    float z = sm_bilinear(val[2 * i], val[2 * i + 1], par + 4 * i);
-    if constexpr (NODE == SLG_NODE_WALSH) z = sm_sigmoid(z);
-    val[NLEAF + i] = z;
+    if constexpr (NODE == SLG_NODE_WALSH) {
+      val[NLEAF + i] = gen_node<NODE, 2>(val + 2 * i, par + 4 * i);
+    } else {  // the forward's on LDS
+      const float* c = par + 4 * i;
+      const float a = val[2 * i], b = val[2 * i + 1];
+      val[NLEAF + i] = fmaf(b, fmaf(a, c[3], c[2]), fmaf(a, c[1], c[0]));
+    }
   }
   float gv[NLEAF + NN];
   gv[NLEAF + NN - 1] = g;
@@ -554,13 +561,13 @@ __device__ inline void sm_window(float (&v)[4][NLEAF], SmWords rc, bool rings,
 }
 
 // The first window position holding the maximum.
-template <int NODE, int NLEAF>
+template <int NODE, int NLEAF, bool LDS = sm_lds_form<NODE>()>
 __device__ inline int sm_first_max(const float (&v)[4][NLEAF], const float* par) {
-  float best = sm_eval<NODE, NLEAF>(v[0], par);
+  float best = sm_eval<NODE, NLEAF, LDS>(v[0], par);
   int qs = 0;
 #pragma unroll
   for (int q = 1; q < 4; ++q) {
-    const float val = sm_eval<NODE, NLEAF>(v[q], par);
+    const float val = sm_eval<NODE, NLEAF, LDS>(v[q], par);
     if (val > best) {
       best = val;
       qs = q;
@@ -571,15 +578,16 @@ __device__ inline int sm_first_max(const float (&v)[4][NLEAF], const float* par)
 
 // Trees whose evaluation and backward together pass the registers: LUTs of 5
 // and 6 leaves (32-64 parameters, 56-112 sums) find their window positions
-// in a launch of their own.
+// in a launch of their own. So do gate16 trees and LUTs whose forward runs
+// through the caches.
 template <int NODE, int NLEAF>
 constexpr bool sm_split() { return !SmTree<NODE, NLEAF>::kBinary && NLEAF >= 5; }
 
 // Window position of every (tree, pooled output, sample): the tree evaluated
-// at the four positions with the forward's operations, the first maximum
-// kept. Two bits per output, the U outputs of a step of a row to a word, route
+// at the four positions with the operations of the forward of its sizes (LDS:
+// sm_eval), the first maximum kept. Two bits per output, the U outputs of a step of a row to a word, route
 // [nc][N][Ho][RW][64].
-template <int NODE, int NLEAF, int KM>
+template <int NODE, int NLEAF, int KM, bool LDS>
 __global__ void __launch_bounds__(64)
 sm_route_kernel(SmArgs a, const uint32_t* __restrict__ recs, const float* __restrict__ xT,
                 uint32_t* __restrict__ route) {
@@ -616,7 +624,7 @@ sm_route_kernel(SmArgs a, const uint32_t* __restrict__ recs, const float* __rest
         if (more) rg.ahead(py, px, nx);
         sm_window<NODE, NLEAF, KM>(v, sm_words(rec), rings, rg, phase,
                                     2 * (py * a.Wp + px) * 256);
-        const int qs = sm_first_max<NODE, NLEAF>(v, NODE == SLG_NODE_HYBRID ? pv : par);
+        const int qs = sm_first_max<NODE, NLEAF, LDS>(v, NODE == SLG_NODE_HYBRID ? pv : par);
         word |= (uint32_t)qs << (2 * u);
         if (++u == a.U || px == a.Wo - 1) {
           rp[(int64_t)(py * a.RW + step++) * 64] = word;
@@ -1142,6 +1150,9 @@ int conv_sm_bwd(const float* x, int64_t B, int64_t C, int64_t H, int64_t W, int6
   SLG_REQUIRE(ws_floats >= p.total, SLG_E_ARG, "conv_soft_bwd: workspace of %lld floats, %lld needed",
               (long long)ws_floats, (long long)p.total);
   SmArgs a = p.a;
+  const bool cache = pool && (node == SLG_NODE_GATE16 || node == SLG_NODE_MULTILINEAR2) &&
+                     !conv_forward_on_lds(C, H, W, N, node, depth, arity, K, pad, pool);
+  a.raw = cache;
   const int64_t nw = N * p.nleaf * K, nn = N * p.nparam;
   uint32_t* recs = reinterpret_cast<uint32_t*>(ws + p.recs);
   int* start = reinterpret_cast<int*>(ws + p.start);
@@ -1168,15 +1179,23 @@ int conv_sm_bwd(const float* x, int64_t B, int64_t C, int64_t H, int64_t W, int6
         const int64_t grid = cdiv(N * a.PS * a.ncg, 8) * 8;
         const int64_t s0 = round * p.a.ncg * a.PS;
         const size_t ring = (size_t)(2 * (a.kernel + 1) * (a.kernel + 1) + 2) * 256;
-        constexpr int kPooled = sm_split<NODE, NL>() ? 2 : 1;
-        if constexpr (kPooled == 2) {
-          if (pool) {
-            hipLaunchKernelGGL((sm_route_kernel<NODE, NL, KM>), dim3((unsigned)grid), dim3(64), ring,
-                               st, a, recs, ws + p.xT, route);
-            SLG_LAUNCH_CHECK("conv_soft_bwd route");
+        constexpr bool kSplit = sm_split<NODE, NL>();
+        constexpr bool kCache = NODE == SLG_NODE_GATE16 || NODE == SLG_NODE_MULTILINEAR2;
+        auto grad = pool ? sm_grad_kernel<NODE, NL, KM, kSplit ? 2 : 1> : sm_grad_kernel<NODE, NL, KM, 0>;
+        void (*find)(SmArgs, const uint32_t*, const float*, uint32_t*) = nullptr;
+        if constexpr (kSplit) {
+          if (pool) find = sm_route_kernel<NODE, NL, KM, true>;
+        }
+        if constexpr (kCache) {
+          if (cache) {
+            find = sm_route_kernel<NODE, NL, KM, false>;
+            grad = sm_grad_kernel<NODE, NL, KM, 2>;
           }
         }
-        auto grad = pool ? sm_grad_kernel<NODE, NL, KM, kPooled> : sm_grad_kernel<NODE, NL, KM, 0>;
+        if (find) {
+          hipLaunchKernelGGL(find, dim3((unsigned)grid), dim3(64), ring, st, a, recs, ws + p.xT, route);
+          SLG_LAUNCH_CHECK("conv_soft_bwd route");
+        }
         hipLaunchKernelGGL(grad, dim3((unsigned)grid), dim3(64), ring, st, a, recs, ws + p.xT,
                            ws + p.gT, route, gl, ws + p.pw + s0 * nw, ws + p.pn + s0 * nn);
         SLG_LAUNCH_CHECK("conv_soft_bwd grad");

@@ -1,7 +1,13 @@
 // The tree of one ConvLogicTree output channel, shared by the soft forward
-// and backward kernels so that both evaluate it with the same operations
-// (the backward's max-pool routing compares the forward's exact values).
+// and backward kernels so that both evaluate it with the same operations:
+// the backward's max-pool routing compares the forward's exact values. There
+// are two forms, rounded differently: conv_tree_eval on the kernels that stage
+// images in LDS, gen_node node by node on the one that reads them through the
+// caches (every walsh tree, deeper trees, larger images); which of the two the
+// forward of given sizes runs is conv_forward_on_lds.
 #pragma once
+
+#include <math.h>
 
 #include "slg_common.h"
 
@@ -96,6 +102,49 @@ __device__ inline float conv_tree_eval(const float (&v)[NLEAF], const float* par
     return t[0];
   }
 }
+
+__device__ inline float tree_sigmoid(float z) { return 1.0f / (1.0f + expf(-z)); }
+
+// Value of one node with children c[0..A) and parameters p, as the forward
+// through the caches evaluates it.
+template <int NODE, int A>
+__device__ inline float gen_node(const float* c, const float* __restrict__ p) {
+  if constexpr (NODE == SLG_NODE_GATE16 || NODE == SLG_NODE_WALSH) {
+    // ((p0 + p1 a) + p2 b) + p3 (a b), three FMAs written out: another
+    // contraction moves the window position of near-ties
+    const float a = c[0], b = c[1];
+    const float z = fmaf(p[3], a * b, fmaf(p[2], b, fmaf(p[1], a, p[0])));
+    if constexpr (NODE == SLG_NODE_WALSH) return tree_sigmoid(z);
+    return z;
+  } else if constexpr (NODE == SLG_NODE_HYBRID) {
+    int addr = 0;
+#pragma unroll
+    for (int j = 0; j < A; ++j) addr |= (c[j] >= 0.5f ? 1 : 0) << j;
+    return p[addr];
+  } else {
+    // the reference's product form (nodes.py:174-178): corner factors a_j or
+    // (1 - a_j) multiplied in leaf order, then sum_p w_p * s_p added in
+    // corner order, each operation rounded on its own (no contraction), so
+    // that values the reference computes as equal (near-ties of a flat tree
+    // at binary leaves) are equal here too: the pooled routing depends on it
+#pragma clang fp contract(off)
+    constexpr int PP = 1 << A;
+    float acc = 0.0f;
+#pragma unroll
+    for (int e = 0; e < PP; ++e) {
+      float w = (e & 1) ? c[0] : 1.0f - c[0];
+#pragma unroll
+      for (int j = 1; j < A; ++j) w = w * ((e >> j) & 1 ? c[j] : 1.0f - c[j]);
+      const float term = w * p[e];
+      acc = e == 0 ? term : acc + term;
+    }
+    return acc;
+  }
+}
+
+// Whether slg_conv_soft_fwd evaluates these trees with conv_tree_eval (conv.hip).
+bool conv_forward_on_lds(int64_t C, int64_t H, int64_t W, int64_t N, int node, int depth, int arity,
+                         int K, int pad, bool pool);
 
 // Node trees on the generic kernels (conv_generic.hip): gate16 and walsh
 // binary trees of depth 1-5, multilinear and hybrid LUT trees with at most
