@@ -219,6 +219,8 @@ def fc_layer(x: Tensor, cand: Tensor, conn: Optional[Tensor], raw: Tensor, node_
     parameters -> ``(y [B,OUT], w [OUT,A,K], npar)``. ``A = 2`` gate16 and
     walsh nodes, and arity-2 multilinear ones, as ``fc_soft``."""
     ops.require_gpu(x, cand, conn, raw)
+    if tuple(raw.shape) != (cand.shape[0], 16 if node_kind == ops.GATE16 else 4):
+        raise ValueError(f"fc_layer: parameters {tuple(raw.shape)} for {cand.shape[0]} outputs")
     cand = ops._c(cand, torch.int32)
     w, npar = ops.layer_params(conn, tuple(cand.shape), [raw], node_kind, 2)
     npar = npar.view(-1, 4)
@@ -271,6 +273,9 @@ def fc_lut_layer(x: Tensor, cand: Tensor, conn: Optional[Tensor], logits: Tensor
     """LUT layer: ``cand/conn [OUT,n,K]``, ``logits [OUT,2^n]`` ->
     ``(y [B,OUT], w, s)``."""
     ops.require_gpu(x, cand, conn, logits)
+    if tuple(logits.shape) != (cand.shape[0], 2 ** cand.shape[1]):
+        raise ValueError(f"fc_lut_layer: logits {tuple(logits.shape)} for candidates "
+                         f"{tuple(cand.shape)}")
     cand = ops._c(cand, torch.int32)
     w, s = ops.layer_params(conn, tuple(cand.shape), [logits], ops.HYBRID, cand.shape[1])
     s = s.view(logits.shape)
@@ -464,8 +469,9 @@ def conv_layer(x: Tensor, conn: Optional[Tensor], l0: Tensor, l1: Optional[Tenso
         # follows the row count, and one bit of a coefficient moves the pooled
         # routing of every near-tie
         w = (torch.ones(cm.shape, device=x.device) if conn is None else
-             torch.softmax(conn, 2))
-        npar = torch.softmax(torch.cat(levels, 1), 2) @ basis
+             torch.softmax(ops._c(conn, torch.float32), 2))
+        gates = torch.cat([ops._c(t, torch.float32) for t in levels], 1)
+        npar = torch.softmax(gates, 2) @ ops._c(basis, torch.float32)
         # autocast runs the product in 16 bits, a default dtype makes the ones
         w, npar = ops._c(w, torch.float32), ops._c(npar, torch.float32)
     else:

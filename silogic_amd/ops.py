@@ -205,9 +205,11 @@ def _level_args(levels, N, P_raw):
     return (ctypes.c_int32 * len(nodes))(*nodes), sum(nodes)
 
 
-def _quads(levels):
-    """Levels at addresses the kernels can read as quads (a traced call's own
-    may be views at any offset, which tracing does not see)."""
+def _levels_f32(levels):
+    """Levels as the kernels read them: contiguous fp32 at addresses of whole
+    quads (a traced call's own may be views at any offset, which tracing does
+    not see, and a direct call's of any type)."""
+    levels = [_c(t, torch.float32) for t in levels]
     return [t if t.data_ptr() % 16 == 0 else t.clone() for t in levels]
 
 
@@ -215,8 +217,10 @@ def layer_params(conn, w_shape, levels, kind, arity, scale=1.0):
     """``(w, npar)`` of a layer from its parameters in one launch: ``w``
     (shape ``[N, ..., K]``) = softmax of ``conn`` (ones for None), ``npar``
     ``[N, nodes, P]`` from the raw parameters of every tree level."""
+    if conn is not None and tuple(conn.shape) != tuple(w_shape):
+        raise ValueError(f"layer_params: conn {tuple(conn.shape)} for candidates {tuple(w_shape)}")
     N, K = w_shape[0], w_shape[-1]
-    levels = _quads(levels)
+    conn, levels = _c(conn, torch.float32), _levels_f32(levels)
     P = 4 if kind in (GATE16, WALSH) else 2 ** arity
     nodes, NN = _level_args(levels, N, 16 if kind == GATE16 else P)
     dev = levels[0].device
@@ -231,7 +235,7 @@ def layer_params_bwd(w, gw, levels, kind, arity, scale, gnp, need_conn, need_lev
     """``(gconn, [level gradients])`` from the gradients of ``w`` and ``npar``
     (None where not needed)."""
     N, K = w.shape[0], w.shape[-1]
-    levels = _quads(levels)
+    levels = _levels_f32(levels)
     P = 4 if kind in (GATE16, WALSH) else 2 ** arity
     nodes, _ = _level_args(levels, N, 16 if kind == GATE16 else P)
     gconn = torch.empty_like(w) if need_conn else None

@@ -136,3 +136,75 @@ def test_operator_takes_parameters_at_any_offset(node):
                                            m.node.kind, 1.0)[0]
         got.append((y.detach(), torch.autograd.grad(y.sum(), shifted)[0]))
     assert all(torch.equal(a, b) for a, b in zip(*got))
+
+
+def _modules():
+    return [sl.LogicLayer(20, 30, node="gate16", k=4, seed=1),
+            sl.LogicLayer(20, 30, node="walsh", k=4, seed=1),
+            sl.LogicLayer(20, 30, node="hybrid", arity=3, k=4, seed=1),
+            sl.ConvLogicTree(3, 5, node="gate16", k=4, seed=1),
+            sl.ConvLogicTree(3, 5, node="walsh", k=4, seed=1),
+            sl.ConvLogicTree(3, 5, node="multilinear", arity=4, k=4, seed=1)]
+
+
+def _operator(m, x, conn, levels):
+    """``m``'s training operator on other parameter tensors."""
+    if isinstance(m, sl.ConvLogicTree):
+        cm, ch, cw = m._taps()
+        gate16 = m.node_name == "gate16"
+        return torch.ops.silogic_hip.conv_layer(
+            x, conn, *levels, *[None] * (5 - len(levels)), m.basis if gate16 else None, cm, ch, cw,
+            m._kind(), m.d, m.node_arity, cm.shape[-1], m.padding, True,
+            1.0 / m.tau if m.node_name == "walsh" else 1.0)[0]
+    cand = m._conn.candidates_i32()
+    if m.is_lut:
+        return torch.ops.silogic_hip.fc_lut_layer(x, cand, conn, levels[0], bool(m.node.hybrid))[0]
+    return torch.ops.silogic_hip.fc_layer(x, cand, conn, levels[0], m.node.kind, m._inv_tau())[0]
+
+
+def _own(m):
+    if isinstance(m, sl.ConvLogicTree):
+        levels = list(m.gate_logits) if m.node_name == "gate16" else [n.raw() for n in m.tree_nodes]
+        return m.conn, levels, torch.rand(3, 3, 6, 8)
+    return m._conn.conn, [m.node.raw()], torch.rand(5, 20)
+
+
+@pytest.mark.parametrize("i", range(6))
+def test_operators_convert_other_layouts_and_types(i):
+    m = _modules()[i].cuda().train()
+    conn, levels, x = _own(m)
+    conn, levels, x = conn.detach(), [t.detach() for t in levels], x.cuda()
+    want = _operator(m, x, conn, levels)
+
+    def strided(t):   # same values, outermost stride 1
+        return t.movedim(0, -1).contiguous().movedim(-1, 0)
+
+    for f in (strided, lambda t: t.double()):
+        args = f(conn).requires_grad_(True), [f(t).requires_grad_(True) for t in levels]
+        y = _operator(m, x, *args)
+        assert torch.equal(y, want)
+        plain = [conn.clone().requires_grad_(True)] + [t.clone().requires_grad_(True) for t in levels]
+        gw = torch.autograd.grad(_operator(m, x, plain[0], plain[1:]).sum(), plain)
+        for g, w, t in zip(torch.autograd.grad(y.sum(), [args[0], *args[1]]), gw, [args[0], *args[1]]):
+            assert g.dtype == t.dtype and torch.equal(g.float(), w)
+
+
+@pytest.mark.parametrize("i", range(6))
+def test_operators_refuse_parameters_of_another_shape(i):
+    # larger tensors: nothing is read past an end, whether or not it is refused
+    m = _modules()[i].cuda().train()
+    conn, levels, x = _own(m)
+    conn, levels, x = conn.detach(), [t.detach() for t in levels], x.cuda()
+    for bad in (torch.cat([conn, conn]), torch.cat([conn, conn], 2), conn.reshape(-1).repeat(2)):
+        with pytest.raises((ValueError, IndexError, RuntimeError)):
+            _operator(m, x, bad, levels)
+    for bad in (torch.cat([levels[0]] * 2), torch.cat([levels[0]] * 2, -1)):
+        with pytest.raises((ValueError, IndexError, RuntimeError)):
+            _operator(m, x, conn, [bad, *levels[1:]])
+
+
+def test_a_layer_with_a_replaced_connection_raises():
+    m = sl.LogicLayer(20, 30, k=4, seed=1).cuda().train()
+    m._conn.conn = torch.nn.Parameter(torch.randn(31, 2, 4, device="cuda"))
+    with pytest.raises(ValueError):
+        m(torch.rand(5, 20).cuda())
