@@ -568,17 +568,21 @@ int slg_conv_tree_hard_prep(const int32_t* cm, const int32_t* ch, const int32_t*
  * 138-143, 174-178): w [rows][K] = softmax of conn's rows (null: ones), and
  * node_param [N][nodes][P], level-major, from raw[i] [N * nodes[i]][16 for
  * gate16, 4 for walsh, 2^arity for LUTs]: gate16 coefficients, walsh
- * coefficients times scale, LUT values. K <= 16, n_levels <= 5; raw levels of
- * gate16 and walsh nodes and node_param 16-byte aligned. */
+ * coefficients times scale, LUT values. probs [N][nodes][16] (null: not
+ * wanted): gate16's softmax, which its backward takes. K <= 16, n_levels <= 5;
+ * raw levels of gate16 and walsh nodes, node_param and probs 16-byte aligned. */
 int slg_layer_params(const float* conn, int64_t rows, int32_t K, int32_t n_levels,
                      const float* const* raw, const int32_t* nodes, int64_t N, int32_t node_kind,
-                     int32_t arity, float scale, float* w, float* node_param, slg_stream_t stream);
-/* The gradients of slg_layer_params' inputs: gconn from (w, gw) (null: not
- * wanted), graw[i] from gnp (graw or a level of it null: not wanted). */
+                     int32_t arity, float scale, float* w, float* node_param, float* probs,
+                     slg_stream_t stream);
+/* The gradients of slg_layer_params' inputs from what it wrote: gconn from
+ * (w, gw) (null: not wanted), graw[i] from gnp (graw or a level of it null:
+ * not wanted) and kept, which is probs for gate16, node_param for LUTs and
+ * unused (null) for walsh nodes. */
 int slg_layer_params_bwd(const float* w, const float* gw, int64_t rows, int32_t K, int32_t n_levels,
-                         const float* const* raw, const int32_t* nodes, int64_t N,
-                         int32_t node_kind, int32_t arity, float scale, const float* gnp,
-                         float* gconn, float* const* graw, slg_stream_t stream);
+                         const int32_t* nodes, int64_t N, int32_t node_kind, int32_t arity,
+                         float scale, const float* kept, const float* gnp, float* gconn,
+                         float* const* graw, slg_stream_t stream);
 
 /* The packed node tree of slg_conv_tree_hard_prep with the 2x2 OR pool
  * fused (pool = 1): xp [C,H,W,nw] -> out [N,Ho/2,Wo/2,nw] or [N,H,W,nw];

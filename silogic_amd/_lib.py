@@ -88,8 +88,8 @@ SIGNATURES = {
     "slg_conv_soft_fwd_records": (C.c_int, [_P, _I64, _I64, _I64, _I64, _I64, _I32, _I32, _I32,
                                             _I32, _P, _I32, _I32, _P, _P]),
     "slg_layer_params": (C.c_int, [_P, _I64, _I32, _I32, _P, _P, _I64, _I32, _I32, _F32, _P, _P,
-                                   _P]),
-    "slg_layer_params_bwd": (C.c_int, [_P, _P, _I64, _I32, _I32, _P, _P, _I64, _I32, _I32, _F32,
+                                   _P, _P]),
+    "slg_layer_params_bwd": (C.c_int, [_P, _P, _I64, _I32, _I32, _P, _I64, _I32, _I32, _F32, _P,
                                        _P, _P, _P, _P]),
     "slg_conv_hard_prep": (C.c_int, [_P, _P, _P, _P, _I64, _I32, _I32, _I32, _I32, _I32, _P, _P,
                                      _P, _P]),

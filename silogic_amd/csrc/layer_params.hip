@@ -23,7 +23,7 @@ struct LpArgs {
   int64_t rows;     // softmax rows of K
   int K;
   int N, NN;        // channels (FC: outputs) and nodes per channel
-  int P, PR;        // kept and raw parameters per node
+  int P;            // kept parameters per node
   int kind, levels;
   float scale;
   int m[kLpLevels], off[kLpLevels];  // nodes per channel of a level, first node id
@@ -97,7 +97,8 @@ __device__ inline float lp_sigmoid(float z) { return 1.0f / (1.0f + expf(-z)); }
 
 __global__ void __launch_bounds__(256) layer_params_kernel(LpArgs a, const float* __restrict__ conn,
                                                            float* __restrict__ w,
-                                                           float* __restrict__ np) {
+                                                           float* __restrict__ np,
+                                                           float* __restrict__ probs) {
   if ((int)blockIdx.x < a.row_blocks) {
     const int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (r >= a.rows) return;
@@ -131,6 +132,12 @@ __global__ void __launch_bounds__(256) layer_params_kernel(LpArgs a, const float
   if (a.kind == SLG_NODE_GATE16) {
     float p[16];
     lp_gate_probs(a.raw[lv] + rr * 16, p);
+    if (probs) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        reinterpret_cast<float4*>(probs + kr * 16)[q] =
+            make_float4(p[4 * q], p[4 * q + 1], p[4 * q + 2], p[4 * q + 3]);
+    }
 #pragma unroll
     for (int i = 0; i < 16; ++i)
 #pragma unroll
@@ -146,9 +153,12 @@ __global__ void __launch_bounds__(256) layer_params_kernel(LpArgs a, const float
   reinterpret_cast<float4*>(np)[kr] = make_float4(c[0], c[1], c[2], c[3]);
 }
 
+// From what the forward wrote: the parameters may have changed since (an
+// update between a forward and its backward).
 __global__ void __launch_bounds__(256)
 layer_params_bwd_kernel(LpArgs a, const float* __restrict__ w, const float* __restrict__ gw,
-                        float* __restrict__ gconn, const float* __restrict__ gnp) {
+                        const float* __restrict__ kept, float* __restrict__ gconn,
+                        const float* __restrict__ gnp) {
   if ((int)blockIdx.x < a.row_blocks) {
     const int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (r >= a.rows) return;
@@ -165,14 +175,21 @@ layer_params_bwd_kernel(LpArgs a, const float* __restrict__ w, const float* __re
   if (!lp_node(a, lut ? t / a.P : t, lv, rr, kr) || !a.graw[lv]) return;
   if (lut) {
     const int e = (int)(t % a.P);
-    const float s = lp_sigmoid(a.raw[lv][rr * a.P + e]);
+    const float s = kept[kr * a.P + e];
     a.graw[lv][rr * a.P + e] = gnp[kr * a.P + e] * (s * (1.0f - s));
     return;
   }
   const float4 g = reinterpret_cast<const float4*>(gnp)[kr];
   if (a.kind == SLG_NODE_GATE16) {
     float p[16], d[16], s = 0.0f;
-    lp_gate_probs(a.raw[lv] + rr * 16, p);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const float4 v = reinterpret_cast<const float4*>(kept + kr * 16)[q];
+      p[4 * q] = v.x;
+      p[4 * q + 1] = v.y;
+      p[4 * q + 2] = v.z;
+      p[4 * q + 3] = v.w;
+    }
     const float gc[4] = {g.x, g.y, g.z, g.w};
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
@@ -194,24 +211,20 @@ layer_params_bwd_kernel(LpArgs a, const float* __restrict__ w, const float* __re
   }
 }
 
-static int lp_args(LpArgs& a, int64_t rows, int32_t K, int32_t n_levels, const float* const* raw,
-                   const int32_t* nodes, int64_t N, int32_t kind, int32_t arity, float scale,
-                   const char* what) {
-  SLG_REQUIRE(raw && nodes, SLG_E_ARG, "%s: null array", what);
+static bool lp_binary(int kind) { return kind == SLG_NODE_GATE16 || kind == SLG_NODE_WALSH; }
+
+static int lp_args(LpArgs& a, int64_t rows, int32_t K, int32_t n_levels, const int32_t* nodes,
+                   int64_t N, int32_t kind, int32_t arity, float scale, const char* what) {
+  SLG_REQUIRE(nodes, SLG_E_ARG, "%s: null array", what);
   SLG_REQUIRE(kind >= SLG_NODE_GATE16 && kind <= SLG_NODE_HYBRID, SLG_E_ARG, "%s: node_kind %d", what,
               kind);
   SLG_REQUIRE(n_levels >= 1 && n_levels <= kLpLevels && K >= 1 && K <= kLpMaxK && arity >= 2 &&
                   arity <= 6 && N > 0 && rows >= 0 && rows < (1LL << 31) && N < (1LL << 28),
               SLG_E_SHAPE, "%s: bad sizes", what);
-  const bool binary = kind == SLG_NODE_GATE16 || kind == SLG_NODE_WALSH;
   a.rows = rows; a.K = K; a.N = (int)N; a.kind = kind; a.levels = n_levels; a.scale = scale;
-  a.P = binary ? 4 : (1 << arity);
-  a.PR = kind == SLG_NODE_GATE16 ? 16 : a.P;
+  a.P = lp_binary(kind) ? 4 : (1 << arity);
   for (int i = 0; i < n_levels; ++i) {
-    SLG_REQUIRE(raw[i] && nodes[i] > 0, SLG_E_ARG, "%s: level %d", what, i);
-    // rows of 4 and 16 values are read as quads
-    SLG_REQUIRE(!binary || (uintptr_t)raw[i] % 16 == 0, SLG_E_ARG, "%s: level %d alignment", what, i);
-    a.raw[i] = raw[i];
+    SLG_REQUIRE(nodes[i] > 0, SLG_E_ARG, "%s: level %d", what, i);
     a.m[i] = nodes[i];
     a.off[i] = a.NN;
     a.NN += nodes[i];
@@ -221,8 +234,7 @@ static int lp_args(LpArgs& a, int64_t rows, int32_t K, int32_t n_levels, const f
 }
 
 static unsigned lp_node_blocks(const LpArgs& a) {
-  const bool lut = a.kind == SLG_NODE_MULTILINEAR2 || a.kind == SLG_NODE_HYBRID;
-  return (unsigned)cdiv((int64_t)a.N * a.NN * (lut ? a.P : 1), 256);
+  return (unsigned)cdiv((int64_t)a.N * a.NN * (lp_binary(a.kind) ? 1 : a.P), 256);
 }
 
 }  // namespace slg
@@ -233,25 +245,33 @@ extern "C" {
 
 int slg_layer_params(const float* conn, int64_t rows, int32_t K, int32_t n_levels,
                      const float* const* raw, const int32_t* nodes, int64_t N, int32_t node_kind,
-                     int32_t arity, float scale, float* w, float* node_param, slg_stream_t stream) {
+                     int32_t arity, float scale, float* w, float* node_param, float* probs,
+                     slg_stream_t stream) {
   LpArgs a{};
-  const int rc = lp_args(a, rows, K, n_levels, raw, nodes, N, node_kind, arity, scale, "layer_params");
+  const int rc = lp_args(a, rows, K, n_levels, nodes, N, node_kind, arity, scale, "layer_params");
   if (rc) return rc;
-  SLG_REQUIRE(w && node_param && (uintptr_t)node_param % 16 == 0, SLG_E_ARG, "layer_params: output");
+  SLG_REQUIRE(raw, SLG_E_ARG, "layer_params: null array");
+  for (int i = 0; i < n_levels; ++i) {
+    // rows of 4 and 16 values are read as quads
+    SLG_REQUIRE(raw[i] && (!lp_binary(node_kind) || (uintptr_t)raw[i] % 16 == 0), SLG_E_ARG,
+                "layer_params: level %d", i);
+    a.raw[i] = raw[i];
+  }
+  SLG_REQUIRE(w && node_param && ((uintptr_t)node_param | (uintptr_t)probs) % 16 == 0, SLG_E_ARG,
+              "layer_params: output");
   a.row_blocks = (int)cdiv(rows, 256);
   hipLaunchKernelGGL(layer_params_kernel, dim3(a.row_blocks + lp_node_blocks(a)), dim3(256), 0,
-                     as_stream(stream), a, conn, w, node_param);
+                     as_stream(stream), a, conn, w, node_param, probs);
   SLG_LAUNCH_CHECK("layer_params");
   return 0;
 }
 
 int slg_layer_params_bwd(const float* w, const float* gw, int64_t rows, int32_t K, int32_t n_levels,
-                         const float* const* raw, const int32_t* nodes, int64_t N,
-                         int32_t node_kind, int32_t arity, float scale, const float* gnp,
-                         float* gconn, float* const* graw, slg_stream_t stream) {
+                         const int32_t* nodes, int64_t N, int32_t node_kind, int32_t arity,
+                         float scale, const float* kept, const float* gnp, float* gconn,
+                         float* const* graw, slg_stream_t stream) {
   LpArgs a{};
-  const int rc =
-      lp_args(a, rows, K, n_levels, raw, nodes, N, node_kind, arity, scale, "layer_params_bwd");
+  const int rc = lp_args(a, rows, K, n_levels, nodes, N, node_kind, arity, scale, "layer_params_bwd");
   if (rc) return rc;
   SLG_REQUIRE(!gconn || (w && gw), SLG_E_ARG, "layer_params_bwd: null weights");
   bool nodes_wanted = false;
@@ -260,13 +280,14 @@ int slg_layer_params_bwd(const float* w, const float* gw, int64_t rows, int32_t 
     a.graw[i] = graw[i];
     nodes_wanted |= graw[i] != nullptr;
   }
-  SLG_REQUIRE(!nodes_wanted || (gnp && (uintptr_t)gnp % 16 == 0), SLG_E_ARG,
-              "layer_params_bwd: node gradients");
+  SLG_REQUIRE(!nodes_wanted || (gnp && (kept || node_kind == SLG_NODE_WALSH) &&
+                                ((uintptr_t)gnp | (uintptr_t)kept) % 16 == 0),
+              SLG_E_ARG, "layer_params_bwd: node gradients");
   a.row_blocks = gconn ? (int)cdiv(rows, 256) : 0;
   const unsigned blocks = a.row_blocks + (nodes_wanted ? lp_node_blocks(a) : 0);
   if (blocks == 0) return 0;
   hipLaunchKernelGGL(layer_params_bwd_kernel, dim3(blocks), dim3(256), 0, as_stream(stream), a, w, gw,
-                     gconn, gnp);
+                     kept, gconn, gnp);
   SLG_LAUNCH_CHECK("layer_params_bwd");
   return 0;
 }

@@ -205,62 +205,72 @@ orpool.register_autograd(_orpool_backward, setup_context=_orpool_setup)
 
 # ---------------------------------------------------------------------------
 # Layers from their own parameters: the training forms of the modules. Each
-# op also returns the weights and node parameters it derived (saved for its
-# backward; not differentiable themselves).
+# op also returns the weights, node parameters and (gate16) gate probabilities
+# it derived: saved for its backward, which reads no parameter again (one may
+# change in place between the two), and not differentiable themselves.
 # ---------------------------------------------------------------------------
-def _layer_outputs(x, y_shape, w_shape, np_shape):
-    return tuple(x.new_empty(s, dtype=torch.float32) for s in (y_shape, w_shape, np_shape))
+def _layer_outputs(x, *shapes):
+    return tuple(x.new_empty(s, dtype=torch.float32) for s in shapes)
+
+
+def _gradients(x, *wanted):
+    """Fake gradients: a shape each, ``[0]`` where it is not needed."""
+    return tuple(x.new_empty(s if n else (0,), dtype=torch.float32) for s, n in wanted)
 
 
 @torch.library.custom_op(f"{_NS}::fc_layer", mutates_args=())
 def fc_layer(x: Tensor, cand: Tensor, conn: Optional[Tensor], raw: Tensor, node_kind: int,
-             inv_tau: float) -> Tuple[Tensor, Tensor, Tensor]:
+             inv_tau: float) -> Tuple[Tensor, Tensor, Tensor, Tensor]:
     """Gate layer: ``x [B,IN]``, ``cand/conn [OUT,A,K]``, ``raw`` the node's
-    parameters -> ``(y [B,OUT], w [OUT,A,K], npar)``. ``A = 2`` gate16 and
-    walsh nodes, and arity-2 multilinear ones, as ``fc_soft``."""
+    parameters -> ``(y [B,OUT], w [OUT,A,K], npar, probs)``. ``A = 2`` gate16
+    and walsh nodes, and arity-2 multilinear ones, as ``fc_soft``; ``probs``
+    ``[OUT,1,16]`` (gate16) or empty."""
     ops.require_gpu(x, cand, conn, raw)
     if tuple(raw.shape) != (cand.shape[0], 16 if node_kind == ops.GATE16 else 4):
         raise ValueError(f"fc_layer: parameters {tuple(raw.shape)} for {cand.shape[0]} outputs")
     cand = ops._c(cand, torch.int32)
-    w, npar = ops.layer_params(conn, tuple(cand.shape), [raw], node_kind, 2)
+    w, npar, probs = ops.layer_params(conn, tuple(cand.shape), [raw], node_kind, 2)
     npar = npar.view(-1, 4)
-    return ops._fc_soft_launch(ops._as_f32(x), cand, w, npar, node_kind, inv_tau), w, npar
+    return ops._fc_soft_launch(ops._as_f32(x), cand, w, npar, node_kind, inv_tau), w, npar, probs
 
 
 @fc_layer.register_fake
 def _(x, cand, conn, raw, node_kind, inv_tau):
-    return _layer_outputs(x, (x.shape[0], cand.shape[0]), cand.shape, (cand.shape[0], 4))
+    OUT = cand.shape[0]
+    return _layer_outputs(x, (x.shape[0], OUT), cand.shape, (OUT, 4),
+                          (OUT, 1, 16) if node_kind == ops.GATE16 else (0,))
 
 
 @torch.library.custom_op(f"{_NS}::fc_layer_bwd", mutates_args=())
-def fc_layer_bwd(x: Tensor, cand: Tensor, raw: Tensor, w: Tensor, npar: Tensor, node_kind: int,
+def fc_layer_bwd(x: Tensor, cand: Tensor, w: Tensor, npar: Tensor, probs: Tensor, node_kind: int,
                  inv_tau: float, gy: Tensor, need_x: bool, need_conn: bool,
                  need_raw: bool) -> Tuple[Tensor, Tensor, Tensor]:
     """``(gx, gconn, graw)`` of fc_layer; unneeded ones are empty."""
     gx, gw, gn = ops.fc_soft_bwd(x, cand, w, npar, node_kind, inv_tau, gy, need_x, need_conn,
                                  need_raw)
-    gconn, (graw,) = ops.layer_params_bwd(w, gw, [raw], node_kind, 2, 1.0, gn, need_conn, [need_raw])
-    return tuple(g if g is not None else _empty(x) for g in (gx, gconn, graw))
+    gconn, (graw,) = ops.layer_params_bwd(w, gw, probs if node_kind == ops.GATE16 else npar, [1],
+                                          node_kind, 2, 1.0, gn, need_conn, [need_raw])
+    return tuple(g if g is not None else _empty(x)
+                 for g in (gx, gconn, None if graw is None else graw.squeeze(1)))
 
 
 @fc_layer_bwd.register_fake
-def _(x, cand, raw, w, npar, node_kind, inv_tau, gy, need_x, need_conn, need_raw):
-    return tuple(x.new_empty(t.shape if n else (0,), dtype=torch.float32)
-                 for t, n in ((x, need_x), (w, need_conn), (raw, need_raw)))
+def _(x, cand, w, npar, probs, node_kind, inv_tau, gy, need_x, need_conn, need_raw):
+    raw = (cand.shape[0], 16 if node_kind == ops.GATE16 else 4)
+    return _gradients(x, (x.shape, need_x), (w.shape, need_conn), (raw, need_raw))
 
 
 def _fc_layer_setup(ctx, inputs, output):
     x, cand, conn, raw, node_kind, inv_tau = inputs
-    ctx.mark_non_differentiable(output[1], output[2])
+    ctx.mark_non_differentiable(*output[1:])
     ctx.set_materialize_grads(False)   # no zero tensors in their place
-    ctx.save_for_backward(x, cand, raw, output[1], output[2])
+    ctx.save_for_backward(x, cand, *output[1:])
     ctx.meta = (node_kind, inv_tau)
 
 
-def _fc_layer_backward(ctx, gy, _gw, _gn):
-    x, cand, raw, w, npar = ctx.saved_tensors
+def _fc_layer_backward(ctx, gy, *_):
     need = ctx.needs_input_grad
-    gx, gc, gr = fc_layer_bwd(x, cand, raw, w, npar, *ctx.meta, gy, need[0], need[2], need[3])
+    gx, gc, gr = fc_layer_bwd(*ctx.saved_tensors, *ctx.meta, gy, need[0], need[2], need[3])
     return _none(gx, need[0]), None, _none(gc, need[2]), _none(gr, need[3]), None, None
 
 
@@ -277,7 +287,7 @@ def fc_lut_layer(x: Tensor, cand: Tensor, conn: Optional[Tensor], logits: Tensor
         raise ValueError(f"fc_lut_layer: logits {tuple(logits.shape)} for candidates "
                          f"{tuple(cand.shape)}")
     cand = ops._c(cand, torch.int32)
-    w, s = ops.layer_params(conn, tuple(cand.shape), [logits], ops.HYBRID, cand.shape[1])
+    w, s, _ = ops.layer_params(conn, tuple(cand.shape), [logits], ops.HYBRID, cand.shape[1])
     s = s.view(logits.shape)
     return ops._fc_lut_launch(ops._as_f32(x), cand, w, s, hybrid), w, s
 
@@ -288,37 +298,35 @@ def _(x, cand, conn, logits, hybrid):
 
 
 @torch.library.custom_op(f"{_NS}::fc_lut_layer_bwd", mutates_args=())
-def fc_lut_layer_bwd(x: Tensor, cand: Tensor, logits: Tensor, w: Tensor, s: Tensor, gy: Tensor,
-                     need_x: bool, need_conn: bool,
-                     need_logits: bool) -> Tuple[Tensor, Tensor, Tensor]:
+def fc_lut_layer_bwd(x: Tensor, cand: Tensor, w: Tensor, s: Tensor, gy: Tensor, need_x: bool,
+                     need_conn: bool, need_logits: bool) -> Tuple[Tensor, Tensor, Tensor]:
     """``(gx, gconn, glogits)`` of fc_lut_layer; unneeded ones are empty."""
     got = ops.fc_lut_soft_bwd(x, cand, w, s, gy, need_x, need_conn, need_logits)
     if got is None:
         raise NotImplementedError("fc_lut_layer backward: the input width exceeds what the "
                                   "kernels stage in LDS")
     gx, gw, gs = got
-    gconn, (gl,) = ops.layer_params_bwd(w, gw, [logits], ops.HYBRID, cand.shape[1], 1.0, gs,
-                                        need_conn, [need_logits])
-    return tuple(g if g is not None else _empty(x) for g in (gx, gconn, gl))
+    gconn, (gl,) = ops.layer_params_bwd(w, gw, s, [1], ops.HYBRID, cand.shape[1], 1.0, gs, need_conn,
+                                        [need_logits])
+    return tuple(g if g is not None else _empty(x)
+                 for g in (gx, gconn, None if gl is None else gl.squeeze(1)))
 
 
 @fc_lut_layer_bwd.register_fake
-def _(x, cand, logits, w, s, gy, need_x, need_conn, need_logits):
-    return tuple(x.new_empty(t.shape if n else (0,), dtype=torch.float32)
-                 for t, n in ((x, need_x), (w, need_conn), (logits, need_logits)))
+def _(x, cand, w, s, gy, need_x, need_conn, need_logits):
+    return _gradients(x, (x.shape, need_x), (w.shape, need_conn), (s.shape, need_logits))
 
 
 def _fc_lut_layer_setup(ctx, inputs, output):
     x, cand, conn, logits, hybrid = inputs
-    ctx.mark_non_differentiable(output[1], output[2])
+    ctx.mark_non_differentiable(*output[1:])
     ctx.set_materialize_grads(False)   # no zero tensors in their place
-    ctx.save_for_backward(x, cand, logits, output[1], output[2])
+    ctx.save_for_backward(x, cand, *output[1:])
 
 
-def _fc_lut_layer_backward(ctx, gy, _gw, _gs):
-    x, cand, logits, w, s = ctx.saved_tensors
+def _fc_lut_layer_backward(ctx, gy, *_):
     need = ctx.needs_input_grad
-    gx, gc, gl = fc_lut_layer_bwd(x, cand, logits, w, s, gy, need[0], need[2], need[3])
+    gx, gc, gl = fc_lut_layer_bwd(*ctx.saved_tensors, gy, need[0], need[2], need[3])
     return _none(gx, need[0]), None, _none(gc, need[2]), _none(gl, need[3]), None
 
 
@@ -457,10 +465,11 @@ def conv_layer(x: Tensor, conn: Optional[Tensor], l0: Tensor, l1: Optional[Tenso
                l2: Optional[Tensor], l3: Optional[Tensor], l4: Optional[Tensor],
                basis: Optional[Tensor], cm: Tensor, ch: Tensor, cw: Tensor, node_kind: int,
                depth: int, arity: int, K: int, pad: int, pool: bool,
-               scale: float) -> Tuple[Tensor, Tensor, Tensor]:
+               scale: float) -> Tuple[Tensor, Tensor, Tensor, Tensor]:
     """Conv tree block from its own parameters (``conn [N,leaves,K]`` and one
     raw tensor per tree level, gate16: the ``basis [16,4]``) -> ``(y, w
-    [N,leaves,K], npar [N,nodes,P])``."""
+    [N,leaves,K], npar [N,nodes,P], probs)``, ``probs`` ``[N,nodes,16]``
+    (gate16) or empty."""
     ops.require_gpu(x, conn, l0, cm)
     cm, ch, cw = (ops._c(t, torch.int32) for t in (cm, ch, cw))
     levels = _levels(l0, l1, l2, l3, l4)
@@ -470,68 +479,71 @@ def conv_layer(x: Tensor, conn: Optional[Tensor], l0: Tensor, l1: Optional[Tenso
         # routing of every near-tie
         w = (torch.ones(cm.shape, device=x.device) if conn is None else
              torch.softmax(ops._c(conn, torch.float32), 2))
-        gates = torch.cat([ops._c(t, torch.float32) for t in levels], 1)
-        npar = torch.softmax(gates, 2) @ ops._c(basis, torch.float32)
+        probs = torch.softmax(torch.cat([ops._c(t, torch.float32) for t in levels], 1), 2)
+        npar = probs @ ops._c(basis, torch.float32)
         # autocast runs the product in 16 bits, a default dtype makes the ones
-        w, npar = ops._c(w, torch.float32), ops._c(npar, torch.float32)
+        w, npar, probs = (ops._c(t, torch.float32) for t in (w, npar, probs))
     else:
-        w, npar = ops.layer_params(conn, tuple(cm.shape), levels, node_kind,
-                                   2 if node_kind == ops.WALSH else arity, scale)
+        w, npar, probs = ops.layer_params(conn, tuple(cm.shape), levels, node_kind,
+                                          2 if node_kind == ops.WALSH else arity, scale)
     y = ops._conv_soft_launch(ops._as_f32(x), npar, w, cm, ch, cw, node_kind, depth, arity, K, pad,
                               pool)
-    return y, w, npar
+    return y, w, npar, probs
 
 
 @conv_layer.register_fake
 def _(x, conn, l0, l1, l2, l3, l4, basis, cm, ch, cw, node_kind, depth, arity, K, pad, pool,
       scale):
     _, nodes, P = ops.tree_shape(node_kind, depth, arity)
-    return _layer_outputs(x, _conv_out_shape(x, cm, pad, pool), cm.shape, (cm.shape[0], nodes, P))
+    N = cm.shape[0]
+    return _layer_outputs(x, _conv_out_shape(x, cm, pad, pool), cm.shape, (N, nodes, P),
+                          (N, nodes, 16) if node_kind == ops.GATE16 else (0,))
 
 
 @torch.library.custom_op(f"{_NS}::conv_layer_bwd", mutates_args=())
-def conv_layer_bwd(x: Tensor, l0: Tensor, l1: Optional[Tensor], l2: Optional[Tensor],
-                   l3: Optional[Tensor], l4: Optional[Tensor], w: Tensor, npar: Tensor, cm: Tensor,
-                   ch: Tensor, cw: Tensor, node_kind: int, depth: int, arity: int, K: int,
+def conv_layer_bwd(x: Tensor, cm: Tensor, ch: Tensor, cw: Tensor, w: Tensor, npar: Tensor,
+                   probs: Tensor, nodes: List[int], node_kind: int, depth: int, arity: int, K: int,
                    pad: int, pool: bool, scale: float, gy: Tensor, need_x: bool, need_conn: bool,
                    need_levels: List[bool]
                    ) -> Tuple[Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor]:
-    """``(gx, gconn, gl0 .. gl4)`` of conv_layer; unneeded ones are empty."""
-    levels = _levels(l0, l1, l2, l3, l4)
+    """``(gx, gconn, gl0 .. gl4)`` of conv_layer, level gradients ``[N,m,P]``;
+    unneeded ones are empty. ``nodes``: m of each level."""
     got = ops.conv_soft_bwd(x, npar, w, cm, ch, cw, node_kind, depth, arity, K, pad, pool, gy, need_x,
                             any(need_levels), need_conn)
     if got is None:
         raise NotImplementedError("conv_layer backward: shape outside the HIP kernels")
     gx, gn, gw = got
-    gconn, gl = ops.layer_params_bwd(w, gw, levels, node_kind,
+    gconn, gl = ops.layer_params_bwd(w, gw, probs if node_kind == ops.GATE16 else npar, nodes, node_kind,
                                      2 if node_kind in (ops.GATE16, ops.WALSH) else arity, scale,
-                                     gn, need_conn, need_levels[:len(levels)])
+                                     gn, need_conn, need_levels[:len(nodes)])
     gl = gl + [None] * (5 - len(gl))
     return tuple(g if g is not None else _empty(x) for g in (gx, gconn, *gl))
 
 
 @conv_layer_bwd.register_fake
-def _(x, l0, l1, l2, l3, l4, w, npar, cm, ch, cw, node_kind, depth, arity, K, pad, pool, scale, gy,
-      need_x, need_conn, need_levels):
-    need = [need_x, need_conn] + list(need_levels)
-    return tuple(x.new_empty(t.shape if n and t is not None else (0,), dtype=torch.float32)
-                 for t, n in zip((x, w, l0, l1, l2, l3, l4), need))
+def _(x, cm, ch, cw, w, npar, probs, nodes, node_kind, depth, arity, K, pad, pool, scale, gy, need_x,
+      need_conn, need_levels):
+    P = 16 if node_kind == ops.GATE16 else npar.shape[-1]
+    shapes = [(w.shape[0], m, P) for m in nodes] + [(0,)] * (5 - len(nodes))
+    return _gradients(x, (x.shape, need_x), (w.shape, need_conn), *zip(shapes, need_levels))
 
 
 def _conv_layer_setup(ctx, inputs, output):
-    x, conn, l0, l1, l2, l3, l4, basis, cm, ch, cw = inputs[:11]
-    ctx.mark_non_differentiable(output[1], output[2])
+    x, conn, l0, l1, l2, l3, l4, basis, cm, ch, cw, node_kind = inputs[:12]
+    ctx.mark_non_differentiable(*output[1:])
     ctx.set_materialize_grads(False)   # no zero tensors in their place
-    ctx.save_for_backward(x, l0, l1, l2, l3, l4, output[1], output[2], cm, ch, cw)
-    ctx.meta = tuple(inputs[11:])
+    ctx.save_for_backward(x, cm, ch, cw, *output[1:])
+    ctx.shapes = [t.shape for t in _levels(l0, l1, l2, l3, l4)]
+    P = 16 if node_kind == ops.GATE16 else output[2].shape[-1]
+    ctx.meta = ([s.numel() // (cm.shape[0] * P) for s in ctx.shapes], *inputs[11:])
 
 
-def _conv_layer_backward(ctx, gy, _gw, _gn):
+def _conv_layer_backward(ctx, gy, *_):
     need = ctx.needs_input_grad
     gx, gc, *gl = conv_layer_bwd(*ctx.saved_tensors, *ctx.meta, gy, need[0], need[1],
                                  [bool(n) for n in need[2:7]])
-    return (_none(gx, need[0]), _none(gc, need[1]),
-            *(_none(g, n) for g, n in zip(gl, need[2:7]))) + (None,) * 11
+    gl = [g.view(s) if n else None for g, n, s in zip(gl, need[2:7], ctx.shapes)]
+    return (_none(gx, need[0]), _none(gc, need[1]), *gl) + (None,) * (16 - len(gl))
 
 
 conv_layer.register_autograd(_conv_layer_backward, setup_context=_conv_layer_setup)

@@ -205,18 +205,22 @@ def _level_args(levels, N, P_raw):
     return (ctypes.c_int32 * len(nodes))(*nodes), sum(nodes)
 
 
+def _quads(t):
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
 def _levels_f32(levels):
     """Levels as the kernels read them: contiguous fp32 at addresses of whole
     quads (a traced call's own may be views at any offset, which tracing does
     not see, and a direct call's of any type)."""
-    levels = [_c(t, torch.float32) for t in levels]
-    return [t if t.data_ptr() % 16 == 0 else t.clone() for t in levels]
+    return [_quads(_c(t, torch.float32)) for t in levels]
 
 
 def layer_params(conn, w_shape, levels, kind, arity, scale=1.0):
-    """``(w, npar)`` of a layer from its parameters in one launch: ``w``
+    """``(w, npar, probs)`` of a layer from its parameters in one launch: ``w``
     (shape ``[N, ..., K]``) = softmax of ``conn`` (ones for None), ``npar``
-    ``[N, nodes, P]`` from the raw parameters of every tree level."""
+    ``[N, nodes, P]`` from the raw parameters of every tree level, ``probs``
+    gate16's softmax ``[N, nodes, 16]`` (other nodes: empty)."""
     if conn is not None and tuple(conn.shape) != tuple(w_shape):
         raise ValueError(f"layer_params: conn {tuple(conn.shape)} for candidates {tuple(w_shape)}")
     N, K = w_shape[0], w_shape[-1]
@@ -226,23 +230,30 @@ def layer_params(conn, w_shape, levels, kind, arity, scale=1.0):
     dev = levels[0].device
     w = torch.empty(w_shape, device=dev, dtype=torch.float32)
     npar = torch.empty((N, NN, P), device=dev, dtype=torch.float32)
+    probs = torch.empty((N, NN, 16) if kind == GATE16 else 0, device=dev, dtype=torch.float32)
     _lib.call("slg_layer_params", _p(conn), w.numel() // K, K, len(levels), _ptrs(levels), nodes, N,
-              kind, arity, float(scale), _p(w), _p(npar), _stream(levels[0]))
-    return w, npar
-
-
-def layer_params_bwd(w, gw, levels, kind, arity, scale, gnp, need_conn, need_levels):
-    """``(gconn, [level gradients])`` from the gradients of ``w`` and ``npar``
-    (None where not needed)."""
-    N, K = w.shape[0], w.shape[-1]
-    levels = _levels_f32(levels)
-    P = 4 if kind in (GATE16, WALSH) else 2 ** arity
-    nodes, _ = _level_args(levels, N, 16 if kind == GATE16 else P)
-    gconn = torch.empty_like(w) if need_conn else None
-    graw = [torch.empty_like(t) if n else None for t, n in zip(levels, need_levels)]
-    _lib.call("slg_layer_params_bwd", _p(w), _p(gw), w.numel() // K, K, len(levels), _ptrs(levels),
-              nodes, N, kind, arity, float(scale), _p(gnp), _p(gconn), _ptrs(graw),
+              kind, arity, float(scale), _p(w), _p(npar), _p(probs) if kind == GATE16 else None,
               _stream(levels[0]))
+    return w, npar, probs
+
+
+def layer_params_bwd(w, gw, kept, nodes, kind, arity, scale, gnp, need_conn, need_levels):
+    """``(gconn, [level gradients [N, m, P]])`` from the gradients of ``w`` and
+    ``npar`` (None where not needed) and what :func:`layer_params` returned,
+    ``kept`` (``probs`` for gate16, ``npar`` for LUTs, unused for walsh):
+    nothing is read from the parameters again, which may have changed since.
+    ``nodes``: nodes per channel of each level."""
+    N, K = w.shape[0], w.shape[-1]
+    P = 16 if kind == GATE16 else 4 if kind == WALSH else 2 ** arity
+    w, kept = _c(w, torch.float32), _quads(_c(kept, torch.float32))
+    if kind != WALSH and kept.numel() != N * sum(nodes) * P:
+        raise ValueError(f"layer_params_bwd: kept {tuple(kept.shape)} for {N} x {nodes} nodes")
+    gconn = torch.empty_like(w) if need_conn else None
+    graw = [torch.empty((N, m, P), device=w.device, dtype=torch.float32) if n else None
+            for m, n in zip(nodes, need_levels)]
+    _lib.call("slg_layer_params_bwd", _p(w), _p(gw), w.numel() // K, K, len(nodes),
+              (ctypes.c_int32 * len(nodes))(*nodes), N, kind, arity, float(scale),
+              None if kind == WALSH else _p(kept), _p(gnp), _p(gconn), _ptrs(graw), _stream(w))
     return gconn, graw
 
 

@@ -208,3 +208,23 @@ def test_a_layer_with_a_replaced_connection_raises():
     m._conn.conn = torch.nn.Parameter(torch.randn(31, 2, 4, device="cuda"))
     with pytest.raises(ValueError):
         m(torch.rand(5, 20).cuda())
+
+
+@pytest.mark.parametrize("data", [False, True], ids=["in-place", "data"])
+@pytest.mark.parametrize("i", range(6))
+def test_an_update_between_forward_and_backward(i, data):
+    # the gradients are those of the parameters the forward ran with
+    m = _modules()[i].cuda().train()
+    conn, levels, x = _own(m)
+    x = x.cuda().requires_grad_(True)
+    call = m.forward_pooled if isinstance(m, sl.ConvLogicTree) else m
+    leaves = [x, conn, *levels]
+    y = call(x)
+    gy = torch.randn(y.shape, generator=torch.Generator().manual_seed(2)).cuda()
+    want = torch.autograd.grad(y, leaves, gy)
+    y = call(x)
+    with torch.no_grad():
+        for p in (conn, *levels):
+            (p.data if data else p).normal_()
+    for got, ref in zip(torch.autograd.grad(y, leaves, gy), want):
+        assert torch.equal(got, ref)
