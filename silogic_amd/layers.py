@@ -137,9 +137,11 @@ class LogicLayer(nn.Module):
 
     def _params_op(self, raw):
         """Whether the layer trains on the operators that take its own
-        parameters (``slg_layer_params``): a plain softmax selection."""
+        parameters (``slg_layer_params``): a plain softmax selection of sizes
+        that the kernels of the backward take (others: the composite one)."""
         conn = self._conn
         return (self.node.plain_softmax() and not getattr(conn, "ste", False)
+                and conn.candidates_i32().numel() < 1 << 31
                 and ops.param_levels_ok(getattr(conn, "conn", None), [raw], conn.k))
 
     def records_ok(self):

@@ -246,8 +246,11 @@ def fc_layer_bwd(x: Tensor, cand: Tensor, w: Tensor, npar: Tensor, probs: Tensor
                  inv_tau: float, gy: Tensor, need_x: bool, need_conn: bool,
                  need_raw: bool) -> Tuple[Tensor, Tensor, Tensor]:
     """``(gx, gconn, graw)`` of fc_layer; unneeded ones are empty."""
-    gx, gw, gn = ops.fc_soft_bwd(x, cand, w, npar, node_kind, inv_tau, gy, need_x, need_conn,
-                                 need_raw)
+    got = ops.fc_soft_bwd(x, cand, w, npar, node_kind, inv_tau, gy, need_x, need_conn, need_raw)
+    if got is None:
+        raise NotImplementedError("fc_layer backward: shape outside the HIP kernels "
+                                  "(K > 16 or 2*OUT*K >= 2^31)")
+    gx, gw, gn = got
     gconn, (graw,) = ops.layer_params_bwd(w, gw, probs if node_kind == ops.GATE16 else npar, [1],
                                           node_kind, 2, 1.0, gn, need_conn, [need_raw])
     return tuple(g if g is not None else _empty(x)
