@@ -213,6 +213,12 @@ def _layer_outputs(x, *shapes):
     return tuple(x.new_empty(s, dtype=torch.float32) for s in shapes)
 
 
+def _output_gradient(ctx, x, gy):
+    """``gy``, or zeros where nothing downstream of the output has a gradient
+    (gradients are not materialized: the other outputs never have one)."""
+    return x.new_zeros(ctx.y_shape, dtype=torch.float32) if gy is None else gy
+
+
 def _gradients(x, *wanted):
     """Fake gradients: a shape each, ``[0]`` where it is not needed."""
     return tuple(x.new_empty(s if n else (0,), dtype=torch.float32) for s, n in wanted)
@@ -267,13 +273,15 @@ def _fc_layer_setup(ctx, inputs, output):
     x, cand, conn, raw, node_kind, inv_tau = inputs
     ctx.mark_non_differentiable(*output[1:])
     ctx.set_materialize_grads(False)   # no zero tensors in their place
+    ctx.y_shape = output[0].shape
     ctx.save_for_backward(x, cand, *output[1:])
     ctx.meta = (node_kind, inv_tau)
 
 
 def _fc_layer_backward(ctx, gy, *_):
-    need = ctx.needs_input_grad
-    gx, gc, gr = fc_layer_bwd(*ctx.saved_tensors, *ctx.meta, gy, need[0], need[2], need[3])
+    need, saved = ctx.needs_input_grad, ctx.saved_tensors
+    gy = _output_gradient(ctx, saved[0], gy)
+    gx, gc, gr = fc_layer_bwd(*saved, *ctx.meta, gy, need[0], need[2], need[3])
     return _none(gx, need[0]), None, _none(gc, need[2]), _none(gr, need[3]), None, None
 
 
@@ -324,12 +332,14 @@ def _fc_lut_layer_setup(ctx, inputs, output):
     x, cand, conn, logits, hybrid = inputs
     ctx.mark_non_differentiable(*output[1:])
     ctx.set_materialize_grads(False)   # no zero tensors in their place
+    ctx.y_shape = output[0].shape
     ctx.save_for_backward(x, cand, *output[1:])
 
 
 def _fc_lut_layer_backward(ctx, gy, *_):
-    need = ctx.needs_input_grad
-    gx, gc, gl = fc_lut_layer_bwd(*ctx.saved_tensors, gy, need[0], need[2], need[3])
+    need, saved = ctx.needs_input_grad, ctx.saved_tensors
+    gy = _output_gradient(ctx, saved[0], gy)
+    gx, gc, gl = fc_lut_layer_bwd(*saved, gy, need[0], need[2], need[3])
     return _none(gx, need[0]), None, _none(gc, need[2]), _none(gl, need[3]), None
 
 
@@ -535,6 +545,7 @@ def _conv_layer_setup(ctx, inputs, output):
     x, conn, l0, l1, l2, l3, l4, basis, cm, ch, cw, node_kind = inputs[:12]
     ctx.mark_non_differentiable(*output[1:])
     ctx.set_materialize_grads(False)   # no zero tensors in their place
+    ctx.y_shape = output[0].shape
     ctx.save_for_backward(x, cm, ch, cw, *output[1:])
     ctx.shapes = [t.shape for t in _levels(l0, l1, l2, l3, l4)]
     P = 16 if node_kind == ops.GATE16 else output[2].shape[-1]
@@ -542,8 +553,9 @@ def _conv_layer_setup(ctx, inputs, output):
 
 
 def _conv_layer_backward(ctx, gy, *_):
-    need = ctx.needs_input_grad
-    gx, gc, *gl = conv_layer_bwd(*ctx.saved_tensors, *ctx.meta, gy, need[0], need[1],
+    need, saved = ctx.needs_input_grad, ctx.saved_tensors
+    gy = _output_gradient(ctx, saved[0], gy)
+    gx, gc, *gl = conv_layer_bwd(*saved, *ctx.meta, gy, need[0], need[1],
                                  [bool(n) for n in need[2:7]])
     gl = [g.view(s) if n else None for g, n, s in zip(gl, need[2:7], ctx.shapes)]
     return (_none(gx, need[0]), _none(gc, need[1]), *gl) + (None,) * (16 - len(gl))

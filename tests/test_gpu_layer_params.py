@@ -228,3 +228,29 @@ def test_an_update_between_forward_and_backward(i, data):
             (p.data if data else p).normal_()
     for got, ref in zip(torch.autograd.grad(y, leaves, gy), want):
         assert torch.equal(got, ref)
+
+
+class _Drop(torch.autograd.Function):
+    """Passes its input on and sends no gradient back."""
+
+    @staticmethod
+    def forward(ctx, y):
+        return y.clone()
+
+    @staticmethod
+    def backward(ctx, g):
+        return None
+
+
+@pytest.mark.parametrize("i", range(6))
+def test_an_output_without_a_gradient_gives_zeros(monkeypatch, i):
+    m = _modules()[i].cuda().train()
+    conn, levels, x = _own(m)
+    call = m.forward_pooled if isinstance(m, sl.ConvLogicTree) else m
+    for on in (True, False):      # the operators, then the torch expressions
+        if not on:
+            monkeypatch.setattr(ops, "param_levels_ok", lambda *a: False)
+        leaves = [x.cuda().requires_grad_(True), conn, *levels]
+        grads = torch.autograd.grad(_Drop.apply(call(leaves[0])).sum(), leaves, allow_unused=True)
+        for g, t in zip(grads, leaves):
+            assert g is not None and g.shape == t.shape and not g.any()
