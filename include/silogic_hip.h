@@ -508,11 +508,17 @@ int slg_conv_soft_fwd_records(const float* x, int64_t B, int64_t C, int64_t H, i
  * and dL/dnode_param into gnp; any of the three may be NULL (not computed).
  * A pooled output's gradient goes to the first window position (row-major)
  * that holds the window's maximum. No atomics on values: every sum runs in
- * a fixed order. Supports every tree slg_conv_soft_fwd takes with K <= 8
- * (gate16 trees of depth 1-3 and depth-1 LUTs on an LDS-staged kernel where
- * the image fits, the others on kernels that read it through the caches);
+ * a fixed order. Supports every tree slg_conv_soft_fwd takes with K <= 8;
  * slg_conv_soft_bwd_workspace returns the workspace floats, or -1 for
- * shapes the kernels do not take. */
+ * shapes the kernels do not take.
+ * The _on forms name the kernels: lanes along samples (binary trees of depth
+ * 1-3, depth-1 LUTs), lanes along output positions (gate16 trees of depth 1-3,
+ * depth-1 LUTs), or those for any tree; AUTO, as the plain forms, takes what is
+ * estimated the shortest. want_gx = 0: the workspace of calls without gx. */
+#define SLG_CONV_BWD_AUTO 0
+#define SLG_CONV_BWD_SAMPLES 1
+#define SLG_CONV_BWD_POSITIONS 2
+#define SLG_CONV_BWD_GENERIC 3
 int64_t slg_conv_soft_bwd_workspace(int64_t B, int64_t C, int64_t H, int64_t W, int64_t N,
                                     int32_t node_kind, int32_t depth, int32_t arity, int32_t K,
                                     int32_t pad, int32_t pool);
@@ -522,6 +528,16 @@ int slg_conv_soft_bwd(const float* x, int64_t B, int64_t C, int64_t H, int64_t W
                       const int32_t* ch, const int32_t* cw, int32_t pad, int32_t pool,
                       const float* gy, float* gx, float* gw, float* gnp, float* workspace,
                       int64_t workspace_floats, slg_stream_t stream);
+
+int64_t slg_conv_soft_bwd_workspace_on(int32_t path, int64_t B, int64_t C, int64_t H, int64_t W,
+                                       int64_t N, int32_t node_kind, int32_t depth, int32_t arity,
+                                       int32_t K, int32_t pad, int32_t pool, int32_t want_gx);
+int slg_conv_soft_bwd_on(int32_t path, const float* x, int64_t B, int64_t C, int64_t H, int64_t W,
+                         int64_t N, int32_t node_kind, int32_t depth, int32_t arity, int32_t K,
+                         const float* node_param, const float* w, const int32_t* cm,
+                         const int32_t* ch, const int32_t* cw, int32_t pad, int32_t pool,
+                         const float* gy, float* gx, float* gw, float* gnp, float* workspace,
+                         int64_t workspace_floats, slg_stream_t stream);
 
 /* Hard conv parameters (layers.py:505-527 + nodes.py:183-189 semantics):
  * leaf (cm,ch,cw) by argmax over conn [N,leaves,K] (conn == NULL: K = 1,

@@ -56,6 +56,10 @@ SIGNATURES = {
                                                 _I32, _I32, _I32]),
     "slg_conv_soft_bwd": (C.c_int, [_P, _I64, _I64, _I64, _I64, _I64, _I32, _I32, _I32, _I32, _P,
                                     _P, _P, _P, _P, _I32, _I32, _P, _P, _P, _P, _P, _I64, _P]),
+    "slg_conv_soft_bwd_workspace_on": (C.c_int64, [_I32, _I64, _I64, _I64, _I64, _I64, _I32, _I32,
+                                                   _I32, _I32, _I32, _I32, _I32]),
+    "slg_conv_soft_bwd_on": (C.c_int, [_I32, _P, _I64, _I64, _I64, _I64, _I64, _I32, _I32, _I32, _I32,
+                                       _P, _P, _P, _P, _P, _I32, _I32, _P, _P, _P, _P, _P, _I64, _P]),
     "slg_fc_lut_soft_workspace": (C.c_int64, [_I64, _I32, _I32]),
     "slg_fc_lut_soft_fwd": (C.c_int, [_P, _I64, _I64, _I64, _I32, _I32, _P, _P, _P, _I32, _P, _P,
                                       _I64, _P]),

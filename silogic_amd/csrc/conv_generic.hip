@@ -535,12 +535,24 @@ static GenBwdPlan gen_bwd_plan(int64_t B, int64_t C, int64_t Hf, int64_t Wf, int
 }
 
 int64_t conv_generic_bwd_workspace(int64_t B, int64_t C, int64_t H, int64_t W, int64_t N, int node,
-                                   int depth, int arity, int K, int pad, bool pool) {
+                                   int depth, int arity, int K, int pad, bool pool, double* us) {
   if (!conv_generic_supported(node, depth, arity)) return -1;
   const int64_t kernel = 2 * pad + 1;
   const int64_t Hf = H + 2 * pad - kernel + 1, Wf = W + 2 * pad - kernel + 1;
   const int64_t Ho = pool ? Hf / 2 : Hf, Wo = pool ? Wf / 2 : Wf;
-  return gen_bwd_plan(B, C, Hf, Wf, N, node, depth, arity, K, Ho, Wo).total();
+  const GenBwdPlan p = gen_bwd_plan(B, C, Hf, Wf, N, node, depth, arity, K, Ho, Wo);
+  if (us) {
+    // Estimated microseconds (conv_bwd.hip): the tap reads and evaluations of a
+    // thread, a pixel's walk over its channel's references, the walk over the
+    // waves' partial sums, the leaf gradients' memory
+    const bool binary = node == SLG_NODE_GATE16 || node == SLG_NODE_WALSH;
+    const int64_t L = conv_generic_leaves(node, depth, arity), NQ = pool ? 4 : 1, cus = device_cus();
+    const int64_t NP = conv_generic_params(node, depth, arity);
+    *us = cdiv(p.nblk * B * N, 8 * cus) * (0.415 * L * K * (NQ + 1) + 0.042 * NP * (NQ + 1) * (binary ? 1 : L)) +
+          1.12 * cdiv(B * C * H * W, 2048 * cus) * ((double)N * L * K / C) + 0.34 * p.slots +
+          2.0e-5 * B * N * L * Ho * Wo;
+  }
+  return p.total();
 }
 
 int conv_generic_bwd(const float* x, int64_t B, int64_t C, int64_t H, int64_t W, int64_t N,

@@ -29,7 +29,7 @@
 // beyond L2: about 350 and 670 MB) at 8-12 waves a CU, which its strips' LDS
 // and registers allow; sm_images the copy rate.
 //
-// Launches, per round of samples (bounded workspace):
+// Launches, per round of samples (kSmRoundFloats):
 //   sm_images    x and gy to sample-minor chunks of 64 samples;
 //   sm_tables    per tree: tap offsets, weights, parameters; per input
 //                channel: its references (tree, leaf, tap) in ascending order;
@@ -313,29 +313,6 @@ __device__ inline SmWords sm_words(const uint32_t* p) {
   return (SmWords)a;
 }
 
-// The tree's value as the forward computes it: on the kernels that stage
-// images in LDS (LDS), or through the caches, node by node. par: the record's.
-template <int NODE, int NLEAF, bool LDS>
-__device__ inline float sm_eval(const float (&v)[NLEAF], const float* par) {
-  if constexpr (LDS) {
-    return conv_tree_eval<NODE, NLEAF>(v, par);
-  } else if constexpr (SmTree<NODE, NLEAF>::kBinary) {
-    float u[NLEAF];
-#pragma unroll
-    for (int l = 0; l < NLEAF; ++l) u[l] = v[l];
-    int nb = 0;
-#pragma unroll
-    for (int cnt = NLEAF; cnt > 1; cnt >>= 1) {
-#pragma unroll
-      for (int m = 0; m < cnt / 2; ++m) u[m] = gen_node<NODE, 2>(u + 2 * m, par + 4 * (nb + m));
-      nb += cnt / 2;
-    }
-    return u[0];
-  } else {
-    return gen_node<NODE, NLEAF>(v, par);
-  }
-}
-
 // Walsh trees have no LDS forward.
 template <int NODE>
 constexpr bool sm_lds_form() { return NODE != SLG_NODE_WALSH; }
@@ -563,11 +540,11 @@ __device__ inline void sm_window(float (&v)[4][NLEAF], SmWords rc, bool rings,
 // The first window position holding the maximum.
 template <int NODE, int NLEAF, bool LDS = sm_lds_form<NODE>()>
 __device__ inline int sm_first_max(const float (&v)[4][NLEAF], const float* par) {
-  float best = sm_eval<NODE, NLEAF, LDS>(v[0], par);
+  float best = tree_eval<NODE, NLEAF, LDS>(v[0], par);
   int qs = 0;
 #pragma unroll
   for (int q = 1; q < 4; ++q) {
-    const float val = sm_eval<NODE, NLEAF, LDS>(v[q], par);
+    const float val = tree_eval<NODE, NLEAF, LDS>(v[q], par);
     if (val > best) {
       best = val;
       qs = q;
@@ -584,9 +561,9 @@ template <int NODE, int NLEAF>
 constexpr bool sm_split() { return !SmTree<NODE, NLEAF>::kBinary && NLEAF >= 5; }
 
 // Window position of every (tree, pooled output, sample): the tree evaluated
-// at the four positions with the operations of the forward of its sizes (LDS:
-// sm_eval), the first maximum kept. Two bits per output, the U outputs of a step of a row to a word, route
-// [nc][N][Ho][RW][64].
+// at the four positions with the operations of the forward of its sizes
+// (tree_eval), the first maximum kept. Two bits per output, the U outputs of a
+// step of a row to a word, route [nc][N][Ho][RW][64].
 template <int NODE, int NLEAF, int KM, bool LDS>
 __global__ void __launch_bounds__(64)
 sm_route_kernel(SmArgs a, const uint32_t* __restrict__ recs, const float* __restrict__ xT,
@@ -1038,7 +1015,7 @@ static constexpr int64_t kSmRoundFloats = int64_t(64) << 20;  // leaf gradients 
 static constexpr int64_t kSmJobs = 4096;                      // waves that fill the chip
 
 static bool sm_plan(int64_t B, int64_t C, int64_t H, int64_t W, int64_t N, int node, int depth,
-                    int arity, int K, int pad, bool pool, SmPlan& p) {
+                    int arity, int K, int pad, bool pool, bool /*want_x*/, SmPlan& p) {
   p = SmPlan{};
   const int rc = sm_dispatch(node, depth, arity, K, [&](auto nd, auto nl, auto km) {
     constexpr int NODE = decltype(nd)::value, NL = decltype(nl)::value, KM = decltype(km)::value;
@@ -1105,11 +1082,37 @@ static bool sm_plan(int64_t B, int64_t C, int64_t H, int64_t W, int64_t N, int n
   return true;
 }
 
+// Estimated microseconds of a call (conv_bwd.hip): serial work of a wave, which
+// the waves of a round share out, per term the tap reads and tree evaluations of
+// sm_grad and sm_route, the window rings of other than 3 x 3 kernels, the steps
+// of sm_gx and the images' copy.
+static double sm_us(const SmPlan& p, bool binary) {
+  const SmArgs& a = p.a;
+  const bool pool = a.Ho != a.H || a.Wo != a.W;
+  const int64_t cus = device_cus(), S = pool ? 2 : 1, NQ = pool ? 4 : 1;
+  const int64_t L = p.nleaf, KM = a.K <= 4 ? 4 : kSmMaxK, rounds = cdiv(p.nc_total, a.nc);
+  const int64_t waves = cdiv((int64_t)a.N * a.PS * a.ncg, 8 * cus);
+  const double outputs = (double)(rounds * waves * a.RPS * a.Wo * cdiv(a.nc, a.ncg));
+  const double ring = pool ? a.kernel + 1 : 0, slow = pool && a.kernel != 3 ? ring * ring : 0;
+  const double grad = outputs * (0.022 * L * KM * (NQ + 1) +
+                                 0.019 * (binary ? 4 * (L - 1) : 1 << L) * (NQ + 1) + 0.32 * ring + 0.11 * slow);
+  const int64_t fit = std::max<int64_t>(1, std::min<int64_t>(16, 160 * 1024 / (((int64_t)a.TH * a.Wp + 1) * 256)));
+  const int64_t strips = cdiv((int64_t)a.C * a.nc * a.nt * a.GS, cus * fit);
+  const int64_t rows = std::min<int64_t>(a.Ho, (a.TH + a.kernel + S - 2) / S + 1);
+  const double refs = (double)a.N * L * a.K / a.C;
+  const double gx = rounds * strips * (refs / a.GS) * cdiv(rows, !pool || a.TH > 2 ? 4 : 3) * a.RW;
+  const double image = (double)p.nc_total * 64 * ((double)a.C * a.Hp * a.Wp + (double)a.N * a.P);
+  return 1.3 + grad + 0.42 * gx + 2.5e-6 * rounds * refs * a.C * a.C + 1.7e-6 * image;
+}
+
 int64_t conv_sm_bwd_workspace(int64_t B, int64_t C, int64_t H, int64_t W, int64_t N, int node,
-                              int depth, int arity, int K, int pad, bool pool) {
+                              int depth, int arity, int K, int pad, bool pool, bool want_x,
+                              double* us) {
   SmPlan p;
-  return sm_plan(std::max<int64_t>(B, 1), C, H, W, N, node, depth, arity, K, pad, pool, p) ? p.total
-                                                                                          : -1;
+  if (!sm_plan(std::max<int64_t>(B, 1), C, H, W, N, node, depth, arity, K, pad, pool, want_x, p))
+    return -1;
+  if (us) *us = sm_us(p, node == SLG_NODE_GATE16 || node == SLG_NODE_WALSH);
+  return p.total;
 }
 
 // sm_gx_kernel for rows in steps of u outputs.
@@ -1141,18 +1144,16 @@ static int sm_sums(const float* pw, const float* pn, int64_t slots, int64_t nw, 
 }
 
 int conv_sm_bwd(const float* x, int64_t B, int64_t C, int64_t H, int64_t W, int64_t N, int node,
-                int depth, int arity, int K, int pad, bool pool, const float* np, const float* w,
-                const int* cm, const int* ch, const int* cw, const float* gy, float* gx, float* gw,
-                float* gnp, float* ws, int64_t ws_floats, hipStream_t st) {
+                int depth, int arity, int K, int pad, bool pool, bool raw, const float* np,
+                const float* w, const int* cm, const int* ch, const int* cw, const float* gy, float* gx,
+                float* gw, float* gnp, float* ws, int64_t ws_floats, hipStream_t st) {
   SmPlan p;
-  SLG_REQUIRE(sm_plan(B, C, H, W, N, node, depth, arity, K, pad, pool, p),
+  SLG_REQUIRE(sm_plan(B, C, H, W, N, node, depth, arity, K, pad, pool, gx != nullptr, p),
               SLG_E_UNSUPPORTED, "conv_soft_bwd: sizes outside the sample-minor kernels");
   SLG_REQUIRE(ws_floats >= p.total, SLG_E_ARG, "conv_soft_bwd: workspace of %lld floats, %lld needed",
               (long long)ws_floats, (long long)p.total);
   SmArgs a = p.a;
-  const bool cache = pool && (node == SLG_NODE_GATE16 || node == SLG_NODE_MULTILINEAR2) &&
-                     !conv_forward_on_lds(C, H, W, N, node, depth, arity, K, pad, pool);
-  a.raw = cache;
+  a.raw = raw;
   const int64_t nw = N * p.nleaf * K, nn = N * p.nparam;
   uint32_t* recs = reinterpret_cast<uint32_t*>(ws + p.recs);
   int* start = reinterpret_cast<int*>(ws + p.start);
@@ -1187,7 +1188,7 @@ int conv_sm_bwd(const float* x, int64_t B, int64_t C, int64_t H, int64_t W, int6
           if (pool) find = sm_route_kernel<NODE, NL, KM, true>;
         }
         if constexpr (kCache) {
-          if (cache) {
+          if (raw) {
             find = sm_route_kernel<NODE, NL, KM, false>;
             grad = sm_grad_kernel<NODE, NL, KM, 2>;
           }

@@ -142,6 +142,30 @@ __device__ inline float gen_node(const float* c, const float* __restrict__ p) {
   }
 }
 
+// The tree's value as the forward computes it: on the kernels that stage
+// images in LDS (LDS), par as conv_tree_eval takes it, or through the caches,
+// node by node, par as the caller's.
+template <int NODE, int NLEAF, bool LDS>
+__device__ inline float tree_eval(const float (&v)[NLEAF], const float* par) {
+  if constexpr (LDS) {
+    return conv_tree_eval<NODE, NLEAF>(v, par);
+  } else if constexpr (NODE == SLG_NODE_GATE16 || NODE == SLG_NODE_WALSH) {
+    float u[NLEAF];
+#pragma unroll
+    for (int l = 0; l < NLEAF; ++l) u[l] = v[l];
+    int nb = 0;
+#pragma unroll
+    for (int cnt = NLEAF; cnt > 1; cnt >>= 1) {
+#pragma unroll
+      for (int m = 0; m < cnt / 2; ++m) u[m] = gen_node<NODE, 2>(u + 2 * m, par + 4 * (nb + m));
+      nb += cnt / 2;
+    }
+    return u[0];
+  } else {
+    return gen_node<NODE, NLEAF>(v, par);
+  }
+}
+
 // Whether slg_conv_soft_fwd evaluates these trees with conv_tree_eval (conv.hip).
 bool conv_forward_on_lds(int64_t C, int64_t H, int64_t W, int64_t N, int node, int depth, int arity,
                          int K, int pad, bool pool);
@@ -159,7 +183,7 @@ int conv_generic_fwd(const float* x, int64_t B, int64_t C, int64_t H, int64_t W,
                      const float* np, const float* w, const int* cm, const int* ch, const int* cw,
                      float* out, int64_t Ho, int64_t Wo, hipStream_t st);
 int64_t conv_generic_bwd_workspace(int64_t B, int64_t C, int64_t H, int64_t W, int64_t N, int node,
-                                   int depth, int arity, int K, int pad, bool pool);
+                                   int depth, int arity, int K, int pad, bool pool, double* us);
 int conv_generic_bwd(const float* x, int64_t B, int64_t C, int64_t H, int64_t W, int64_t N,
                      int node, int depth, int arity, int K, int pad, bool pool, const float* np,
                      const float* w, const int* cm, const int* ch, const int* cw, const float* gy,

@@ -984,18 +984,22 @@ def conv_soft_bwd_supported(x, cm, node_kind, depth, arity, K, pad, pool):
                                                   arity, K, pad, int(bool(pool))) >= 0
 
 
+# the kernels of the conv backward (SLG_CONV_BWD_*)
+CONV_BWD_AUTO, CONV_BWD_SAMPLES, CONV_BWD_POSITIONS, CONV_BWD_GENERIC = range(4)
+
+
 def conv_soft_bwd(x, npar, w, cm, ch, cw, node_kind, depth, arity, K, pad, pool, gy,
-                  need_x=True, need_np=True, need_w=True):
+                  need_x=True, need_np=True, need_w=True, path=CONV_BWD_AUTO):
     """HIP backward of the conv soft op: ``(gx, gnp, gw)`` (None where not
-    needed), or None when the kernel does not take the shape."""
+    needed), or None when the kernels (``path``: which) do not take the shape."""
     require_gpu(x, npar, w, cm, gy)
     x = _as_f32(x.detach())
     npar, w = _c(npar.detach(), torch.float32), _c(w.detach(), torch.float32)
     cm, ch, cw = _c(cm, torch.int32), _c(ch, torch.int32), _c(cw, torch.int32)
     B, Cc, H, W = x.shape
     N = cm.shape[0]
-    ws = _lib.lib().slg_conv_soft_bwd_workspace(B, Cc, H, W, N, node_kind, depth, arity, K, pad,
-                                                int(bool(pool)))
+    ws = _lib.lib().slg_conv_soft_bwd_workspace_on(path, B, Cc, H, W, N, node_kind, depth, arity, K,
+                                                   pad, int(bool(pool)), int(need_x))
     if ws < 0:
         return None
     gy = _c(gy, torch.float32)
@@ -1003,7 +1007,7 @@ def conv_soft_bwd(x, npar, w, cm, ch, cw, node_kind, depth, arity, K, pad, pool,
     gn = torch.empty_like(npar) if need_np else None
     gw = torch.empty_like(w) if need_w else None
     work = torch.empty(max(ws, 1), device=x.device, dtype=torch.float32)
-    _lib.call("slg_conv_soft_bwd", _p(x), B, Cc, H, W, N, node_kind, depth, arity, K, _p(npar),
+    _lib.call("slg_conv_soft_bwd_on", path, _p(x), B, Cc, H, W, N, node_kind, depth, arity, K, _p(npar),
               _p(w), _p(cm), _p(ch), _p(cw), pad, int(bool(pool)), _p(gy), _p(gx), _p(gw),
               _p(gn), _p(work), ws, _stream(x))
     return gx, gn, gw
