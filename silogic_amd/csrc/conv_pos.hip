@@ -622,7 +622,7 @@ static int next_pow2(int v) {
 
 template <int NODE, int NLEAF, bool POOL>
 static bool pos_plan_t(int64_t B, int64_t C, int64_t H, int64_t W, int64_t N, int K, int pad,
-                       int64_t Ho, int64_t Wo, bool raw, bool /*want_x*/, PosPlan& p) {
+                       int64_t Ho, int64_t Wo, bool raw, bool want_x, PosPlan& p) {
   using Nd = ConvNode<NODE, NLEAF>;
   const int64_t CHW = C * H * W, P = Ho * Wo;
   const int64_t cap = std::min<int64_t>(device_lds_bytes(), 160 * 1024);
@@ -681,7 +681,7 @@ static bool pos_plan_t(int64_t B, int64_t C, int64_t H, int64_t W, int64_t N, in
   p.keys_ints = (p.R + 3) & ~3LL;
   p.table_ints = ref_table_ints(p.R, nkeys);
   p.ent_ints = 4 * p.R;
-  p.partx_floats = p.NG > 1 ? (((int64_t)p.NG * B * CHW + 3) & ~3LL) : 0;
+  p.partx_floats = p.NG > 1 && want_x ? (((int64_t)p.NG * B * CHW + 3) & ~3LL) : 0;
   p.partw_floats = ((int64_t)p.NR * N * NLEAF * K + 3) & ~3LL;
   p.partn_floats = ((int64_t)p.NR * N * Nd::NP + 3) & ~3LL;
   return true;

@@ -1011,11 +1011,13 @@ struct SmPlan {
   int64_t recs, start, refs, xT, gT, route, gl, pw, pn, parts, total;
 };
 
-static constexpr int64_t kSmRoundFloats = int64_t(64) << 20;  // leaf gradients of a round
+// A round's leaf gradients and its workspace in floats, at most, or one chunk
+// of 64 samples whatever that takes.
+static constexpr int64_t kSmRoundLeaves = int64_t(64) << 20, kSmRoundFloats = int64_t(96) << 20;
 static constexpr int64_t kSmJobs = 4096;                      // waves that fill the chip
 
 static bool sm_plan(int64_t B, int64_t C, int64_t H, int64_t W, int64_t N, int node, int depth,
-                    int arity, int K, int pad, bool pool, bool /*want_x*/, SmPlan& p) {
+                    int arity, int K, int pad, bool pool, bool want_x, SmPlan& p) {
   p = SmPlan{};
   const int rc = sm_dispatch(node, depth, arity, K, [&](auto nd, auto nl, auto km) {
     constexpr int NODE = decltype(nd)::value, NL = decltype(nl)::value, KM = decltype(km)::value;
@@ -1045,7 +1047,8 @@ static bool sm_plan(int64_t B, int64_t C, int64_t H, int64_t W, int64_t N, int n
   a.xs = a.Cz * Hp * Wp * 64;
   p.nc_total = cdiv(B, 64);
   const int64_t gl1 = N * p.nleaf * P * 64;
-  a.nc = (int)std::max<int64_t>(1, std::min<int64_t>(p.nc_total, kSmRoundFloats / gl1));
+  const int64_t chunk = gl1 + a.xs + N * (P + Ho * a.RW) * 64;  // with its images and routes
+  a.nc = (int)std::max<int64_t>(1, std::min({p.nc_total, kSmRoundLeaves / gl1, kSmRoundFloats / chunk}));
   // rows split until the jobs fill the chip; then several chunks to a job
   a.PS = (int)std::max<int64_t>(1, std::min<int64_t>(Ho, cdiv(kSmJobs, N * a.nc)));
   a.RPS = (int)cdiv(Ho, a.PS);
@@ -1068,16 +1071,18 @@ static bool sm_plan(int64_t B, int64_t C, int64_t H, int64_t W, int64_t N, int n
     o += sm_round(words);
     return at;
   };
+  // the rounds do not follow want_x: the weight sums keep their order (and bits)
+  const int64_t gx = want_x;
   p.recs = take(N * p.rec_words);
-  p.start = take(C + 1);
-  p.refs = take((N * p.nleaf * K + 1) * 4);
+  p.start = take(gx * (C + 1));
+  p.refs = take(gx * (N * p.nleaf * K + 1) * 4);
   p.xT = take(a.nc * a.xs);
   p.gT = take(a.nc * N * P * 64);
   p.route = take(pool ? a.nc * N * Ho * a.RW * 64 : 0);
-  p.gl = take(a.nc * gl1);
+  p.gl = take(gx * a.nc * gl1);
   p.pw = take(p.slots * N * p.nleaf * K);
   p.pn = take(p.slots * N * p.nparam);
-  p.parts = take((a.GS - 1) * std::min<int64_t>(B, a.nc * int64_t(64)) * C * H * W);
+  p.parts = take(gx * (a.GS - 1) * std::min<int64_t>(B, a.nc * int64_t(64)) * C * H * W);
   p.total = o;
   return true;
 }

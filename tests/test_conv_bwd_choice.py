@@ -35,6 +35,23 @@ def test_conv_backward_takes_the_shorter_kernels(paths, size):
     assert got not in others
 
 
+def test_a_call_without_input_gradient_reserves_none():
+    size = (512, 3, 32, 64, ops.GATE16, 2, 2, 4, 1, 1)
+    with_gx, without = _floats(AUTO, *size), _floats(AUTO, *size, 0)
+    leaf_gradients = 512 * 64 * 4 * 16 * 16
+    assert with_gx - without >= leaf_gradients
+    assert with_gx == _lib.lib().slg_conv_soft_bwd_workspace(512, 3, 32, 32, *size[3:])
+
+
+@pytest.mark.parametrize("size", [
+    (65536, 512, 8, 8, ops.GATE16, 2, 2, 4, 1, 1),       # few trees under many channels
+    (4096, 64, 32, 512, ops.MULTILINEAR2, 1, 6, 4, 1, 1),
+])
+def test_rounds_bound_the_workspace(size):
+    # 96 M floats of a round, the partial sums of its jobs and the tables
+    assert 0 < _floats(SAMPLES, *size) < 112 << 20
+
+
 def test_refusals():
     size = (4, 3, 8, 4, ops.WALSH, 2, 2, 4, 1, 1)
     assert _floats(POSITIONS, *size) == -1 and _floats(4, *size) == -1 and _floats(-1, *size) == -1
