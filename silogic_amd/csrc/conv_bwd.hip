@@ -9,11 +9,12 @@
 // along samples / positions / generic: gate16 depth 2, K = 4: 759 / 352 / 113
 // us; 16 of them: 676 / 389 / 547; 64 -> 128, 3 x 3, 14 x 14, 256 samples: 114 /
 // 297 / 580. No one size divides them, so each file estimates its time from what
-// it would launch, and the shortest is taken. The terms' factors were fitted to
-// 1900 random shapes (1-1024 samples, 1-512 channels, maps of 4-128, kernels
-// 1-7, every node kind, with and without pooling): the estimates scatter by
-// about 30%, the choice is within 3% of the best of the three for nine in ten
-// and 1.5% slower than it on average. Not by whether the input gradient is
+// it would launch, and the shortest is taken. The factors were fitted to 4700
+// random shapes (1-1024 samples, 1-512 channels, maps of 4-128, kernels 1-7,
+// every node kind, pooled and not, each timed on all three): the estimates
+// scatter by 25-30%; the choice is 1.8% slower than the best of the three on
+// average, one call in twenty by more than 10%, the worst 2.9 times (always along
+// samples: 18% on average, 20 times). Not by whether the input gradient is
 // wanted: the other gradients are the same bits with and without it.
 #include "conv_pos.h"
 #include "conv_sm.h"
@@ -45,8 +46,8 @@ static ConvBwdChoice conv_bwd_choose(int path, int64_t B, int64_t C, int64_t H, 
   };
   c.path = path;
   if (path == SLG_CONV_BWD_AUTO) {
-    // past 1 GB of workspace only where no other kernels take the sizes
-    constexpr int64_t kMost = int64_t(256) << 20;
+    // past 4 GB of workspace only where no other kernels take the sizes
+    constexpr int64_t kMost = int64_t(1) << 30;
     double best = 0.0;
     bool best_large = false;
     for (int p = SLG_CONV_BWD_SAMPLES; p <= SLG_CONV_BWD_GENERIC; ++p) {

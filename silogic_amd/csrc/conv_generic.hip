@@ -542,15 +542,17 @@ int64_t conv_generic_bwd_workspace(int64_t B, int64_t C, int64_t H, int64_t W, i
   const int64_t Ho = pool ? Hf / 2 : Hf, Wo = pool ? Wf / 2 : Wf;
   const GenBwdPlan p = gen_bwd_plan(B, C, Hf, Wf, N, node, depth, arity, K, Ho, Wo);
   if (us) {
-    // Estimated microseconds (conv_bwd.hip): the tap reads and evaluations of a
-    // thread, a pixel's walk over its channel's references, the walk over the
-    // waves' partial sums, the leaf gradients' memory
+    // Estimated microseconds of a call that wants every gradient (conv_bwd.hip):
+    // the tap reads and evaluations of a thread and of all on the chip, a pixel's
+    // walk over its channel's references, the partial sums' over the waves, memory
     const bool binary = node == SLG_NODE_GATE16 || node == SLG_NODE_WALSH;
-    const int64_t L = conv_generic_leaves(node, depth, arity), NQ = pool ? 4 : 1, cus = device_cus();
-    const int64_t NP = conv_generic_params(node, depth, arity);
-    *us = cdiv(p.nblk * B * N, 8 * cus) * (0.415 * L * K * (NQ + 1) + 0.042 * NP * (NQ + 1) * (binary ? 1 : L)) +
-          1.12 * cdiv(B * C * H * W, 2048 * cus) * ((double)N * L * K / C) + 0.34 * p.slots +
-          2.0e-5 * B * N * L * Ho * Wo;
+    const int64_t L = conv_generic_leaves(node, depth, arity), NP = conv_generic_params(node, depth, arity);
+    const double tap = (double)L * K * (pool ? 5 : 1), eval = (double)NP * (pool ? 5 : 1) * (binary ? 1 : L);
+    const double all = (double)(p.nblk * B * N) / (8 * device_cus());
+    const double refs = (double)N * L * K / C;
+    *us = 7 + (0.33 + 0.68 * all) * tap + (0.016 + 0.038 * all) * eval +
+          refs * (1.1 + 1.8e-6 * B * C * H * W) + p.slots * (0.36 + 4e-5 * N * (NP + 8 * L)) +
+          1.5e-6 * B * N * L * H * W;
   }
   return p.total();
 }

@@ -752,22 +752,26 @@ int64_t conv_pos_bwd_workspace(int64_t B, int64_t C, int64_t H, int64_t W, int64
     constexpr bool LUT = NODE != SLG_NODE_GATE16;
     n = p.total();
     if (!us) return;
-    // Estimated microseconds (conv_bwd.hip): what a workgroup does one after the
-    // other: a thread's tap reads, a wave's pixels and references, the image's
-    // staging; then the groups' images
-    const int64_t HW = H * W, P = decltype(pl)::value ? (H / 2) * (W / 2) : HW;
-    const int64_t NQ = decltype(pl)::value ? 4 : 1;
+    // Estimated microseconds of a call that wants every gradient (conv_bwd.hip)
+    constexpr bool POOL = decltype(pl)::value;
+    constexpr int NC1 = 1 << (NL / 2), NC2 = 1 << (NL - NL / 2);
+    const int64_t HW = H * W, P = POOL ? (H / 2) * (W / 2) : HW;
     const int64_t per_cu = std::max<int64_t>(
         1, std::min<int64_t>(2048 / p.threads, (int64_t)(160 * 1024) / (int64_t)p.lds));
-    const double samples = (double)cdiv((int64_t)p.NG * p.NR, device_cus() * per_cu) * p.SPR;
+    // the samples of a workgroup, one after the other, and all on the chip
+    const double own = p.SPR, all = (double)p.NG * p.NR / (device_cus() * per_cu) * p.SPR;
+    const double most = std::max(own, all);
+    // a thread's tap reads, a wave's references and buckets, the image's staging
+    const double tap = (double)cdiv(P, p.TPT) * NL * K * (POOL ? 5 : 1);
     const int64_t ppl = std::min<int64_t>(LUT && NL >= 5 ? 2 : 4, cdiv(HW, 64));
     const double chunks = (double)cdiv(C * cdiv(HW, 64 * ppl), p.threads / 64);
-    const double refs = (double)p.TG * NL * K / C;
-    *us = 27 + samples * (cdiv(P, p.TPT) * (0.235 * NL * K * (NQ + 1) + 0.03) +
-                          chunks * (0.08 * refs * ppl + 0.33 * p.KB) +
-                          (p.XS ? 0.3 * C * HW / p.threads : 0.0)) +
-          (p.NG > 1 ? 2.4e-6 * p.NG * B * C * HW : 0.0) +
-          0.08 * (NL * (K <= 4 ? 4 : kPosMaxK) + ConvNode<NODE, NL>::NP);
+    const double refs = (double)p.TG * NL * K / C, stage = p.XS ? (double)C * HW / p.threads : 0;
+    // LUT corners of the positions; the sums over a tree's threads at the end
+    const double corners = LUT ? (double)P * NC2 * cdiv(p.TG * NC1 * p.J2, p.threads) / p.J2 : 0;
+    const double sums = NL * K + (LUT ? 0 : ConvNode<NODE, NL>::NP);
+    *us = 25 + own * (0.14 * tap + chunks * (0.098 * refs * ppl + 0.19 * p.KB) + 0.15 * stage) +
+          all * (0.041 * tap + 0.54 * stage) + most * ((p.XS ? 0 : 0.065) * tap + 0.052 * corners) +
+          sums * (2.4 + 0.0059 * p.TPT) + (p.NG > 1 ? 1.5e-6 * p.NG * B * C * HW : 0.0);
   });
   return n;
 }

@@ -1087,27 +1087,32 @@ static bool sm_plan(int64_t B, int64_t C, int64_t H, int64_t W, int64_t N, int n
   return true;
 }
 
-// Estimated microseconds of a call (conv_bwd.hip): serial work of a wave, which
-// the waves of a round share out, per term the tap reads and tree evaluations of
-// sm_grad and sm_route, the window rings of other than 3 x 3 kernels, the steps
-// of sm_gx and the images' copy.
-static double sm_us(const SmPlan& p, bool binary) {
+// Estimated microseconds of a call that wants every gradient (conv_bwd.hip).
+static double sm_us(const SmPlan& p, bool binary, bool pool) {
   const SmArgs& a = p.a;
-  const bool pool = a.Ho != a.H || a.Wo != a.W;
-  const int64_t cus = device_cus(), S = pool ? 2 : 1, NQ = pool ? 4 : 1;
-  const int64_t L = p.nleaf, KM = a.K <= 4 ? 4 : kSmMaxK, rounds = cdiv(p.nc_total, a.nc);
-  const int64_t waves = cdiv((int64_t)a.N * a.PS * a.ncg, 8 * cus);
-  const double outputs = (double)(rounds * waves * a.RPS * a.Wo * cdiv(a.nc, a.ncg));
-  const double ring = pool ? a.kernel + 1 : 0, slow = pool && a.kernel != 3 ? ring * ring : 0;
-  const double grad = outputs * (0.022 * L * KM * (NQ + 1) +
-                                 0.019 * (binary ? 4 * (L - 1) : 1 << L) * (NQ + 1) + 0.32 * ring + 0.11 * slow);
-  const int64_t fit = std::max<int64_t>(1, std::min<int64_t>(16, 160 * 1024 / (((int64_t)a.TH * a.Wp + 1) * 256)));
-  const int64_t strips = cdiv((int64_t)a.C * a.nc * a.nt * a.GS, cus * fit);
+  const int S = pool ? 2 : 1, visits = pool ? 5 : 1, L = p.nleaf;
+  const double cus = device_cus(), rounds = (double)cdiv(p.nc_total, a.nc), chunks = (double)p.nc_total;
+  const double taps = (double)a.N * L * a.K, refs = taps / a.C;
+  // sm_grad and sm_route, per output: tap reads and evaluations at the window
+  // positions and the routed one, the window ring's new columns (those of other
+  // than 3 x 3 kernels four loads at a time). The outputs of a wave, one after
+  // the other, and all of them on the chip's waves.
+  const double tap = L * (a.K <= 4 ? 4 : kSmMaxK) * visits, eval = (binary ? 4 * (L - 1) : 1 << L) * visits;
+  const double ring = pool ? a.kernel + 1 : 0, slow = a.kernel == 3 ? 0 : ring * (a.kernel + 1);
+  const double own = rounds * a.RPS * a.Wo * cdiv(a.nc, a.ncg);
+  const double all = (double)a.N * a.P * chunks / (8 * cus);
+  const double grad = own * (0.025 * tap + 0.018 * eval + 0.26 * ring + 0.076 * slow) +
+                      all * (0.0092 * eval + 0.31 * ring + 0.097 * slow);
+  // sm_gx: a wave's references times its steps over the map, and all of them
+  const int64_t resident = std::min<int64_t>(16, 160 * 1024 / (((int64_t)a.TH * a.Wp + 1) * 256));
   const int64_t rows = std::min<int64_t>(a.Ho, (a.TH + a.kernel + S - 2) / S + 1);
-  const double refs = (double)a.N * L * a.K / a.C;
-  const double gx = rounds * strips * (refs / a.GS) * cdiv(rows, !pool || a.TH > 2 ? 4 : 3) * a.RW;
-  const double image = (double)p.nc_total * 64 * ((double)a.C * a.Hp * a.Wp + (double)a.N * a.P);
-  return 1.3 + grad + 0.42 * gx + 2.5e-6 * rounds * refs * a.C * a.C + 1.7e-6 * image;
+  const double steps = rounds * (refs / a.GS) * cdiv(rows, !pool || a.TH > 2 ? 4 : 3) * a.RW;
+  const double waves = (double)a.C * a.nc * a.nt * a.GS / (cus * std::max<int64_t>(1, resident));
+  const double gx = steps * (0.22 * (1 + 3 / sqrt(refs)) + 0.19 * waves);
+  const double tables = 1e-6 * rounds * a.C * taps + 2.4e-3 * taps;
+  const double memory = 64e-6 * chunks * (1.4 * ((double)a.C * a.Hp * a.Wp + (double)a.N * a.P) +
+                                          1.3 * (double)a.N * L * a.P);
+  return 1.5 + 2 * rounds + grad + gx + tables + memory;
 }
 
 int64_t conv_sm_bwd_workspace(int64_t B, int64_t C, int64_t H, int64_t W, int64_t N, int node,
@@ -1116,7 +1121,7 @@ int64_t conv_sm_bwd_workspace(int64_t B, int64_t C, int64_t H, int64_t W, int64_
   SmPlan p;
   if (!sm_plan(std::max<int64_t>(B, 1), C, H, W, N, node, depth, arity, K, pad, pool, want_x, p))
     return -1;
-  if (us) *us = sm_us(p, node == SLG_NODE_GATE16 || node == SLG_NODE_WALSH);
+  if (us) *us = sm_us(p, node == SLG_NODE_GATE16 || node == SLG_NODE_WALSH, pool);
   return p.total;
 }
 
