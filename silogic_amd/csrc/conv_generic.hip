@@ -112,70 +112,95 @@ __device__ inline void gen_eval(float* val, const float* __restrict__ par) {
 // B = 256, pooled: 210 -> 68 us, against one workgroup per sample, channel
 // and 256 positions with a tap's positions read one after the other. Depth 5
 // (one at a time), 16 -> 64 at 16x16, B = 128: 578 -> 423 us a call.
-template <int NODE, int A, int D, int NQ>
+// NARROW: a workgroup's images and outputs within 4 GB of its first sample's,
+// positions below 2^24: 32-bit offsets from uniform bases and divisions by
+// reciprocals. A workgroup takes cpw channels of its run.
+template <int NODE, int A, int D, int NQ, bool NARROW>
 __global__ void __launch_bounds__(256)
 conv_generic_fwd_kernel(const float* __restrict__ x, int C, int H, int W, int N, int K, int kernel,
-                        int pad, int pool, int Ho, int Wo, int64_t total, int64_t nwork,
+                        int pad, int pool, int Ho, int Wo, float inv_hw, float inv_w, int64_t total,
+                        int64_t nwork, int groups, float inv_n, int cpw,
                         const float* __restrict__ np, const float* __restrict__ w,
                         const int* __restrict__ cm, const int* __restrict__ ch,
                         const int* __restrict__ cw, float* __restrict__ out) {
   using T = GenTree<NODE, A, D>;
   const int HoWo = Ho * Wo;
   for (int64_t id = xcd_logical_id(blockIdx.x, gridDim.x); id < nwork; id += gridDim.x) {
-    const int64_t run = id / N;
-    const int n = (int)(id - run * N);
+    const int64_t run = NARROW ? div_small((int)id, groups, inv_n) : id / groups;
+    const int n0 = __builtin_amdgcn_readfirstlane((int)(id - run * groups)) * cpw;
     const int64_t g0 = run * 256;
-    const int64_t b0 = g0 / HoWo;
-    const uint32_t r = (uint32_t)(g0 - b0 * HoWo) + threadIdx.x;
-    const uint32_t db = r / (uint32_t)HoWo;
-    const int p = (int)(r - db * (uint32_t)HoWo);
+    int64_t b0;
+    if (NARROW && HoWo >= 256) {  // a quotient of at most 2^23, within 2 of the true one
+      int q = (int)((float)(int)g0 * inv_hw), e = (int)g0 - q * HoWo;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int d = (e >= HoWo) - (e < 0);
+        q += d;
+        e -= d * HoWo;
+      }
+      b0 = q;
+    } else {
+      b0 = NARROW ? (int64_t)((uint32_t)g0 / (uint32_t)HoWo) : g0 / HoWo;
+    }
+    const int r = (int)(g0 - b0 * HoWo) + (int)threadIdx.x;
+    const int db = NARROW ? div_small(r, HoWo, inv_hw) : r / HoWo;
+    const int p = r - db * HoWo;
     if (g0 + threadIdx.x >= total) continue;
-    const int64_t b = b0 + db;
-    const int oy = p / Wo, ox = p - (p / Wo) * Wo;
-    const float* xb = x + b * C * H * W;
-    const float* par = np + (int64_t)n * T::NN * T::P;
-    float best = -INFINITY;
-    const int nq = pool ? 4 : 1;
-    for (int q0 = 0; q0 < nq; q0 += NQ) {
-      const int y0 = (pool ? 2 * oy + (q0 >> 1) : oy) - pad;
-      const int x0 = (pool ? 2 * ox + (q0 & 1) : ox) - pad;
-      float lv[NQ][T::NLEAF];
+    const int oy = NARROW ? div_small(p, Wo, inv_w) : p / Wo, ox = p - oy * Wo;
+    const float* xb = x + (b0 + (NARROW ? 0 : db)) * C * H * W;
+    const uint32_t xo = NARROW ? (uint32_t)db * (uint32_t)(C * H * W) : 0u;
+    for (int n = n0; n < min(n0 + cpw, N); ++n) {
+      const float* par = np + (int64_t)n * T::NN * T::P;
+      float best = -INFINITY;
+      const int nq = pool ? 4 : 1;
+      for (int q0 = 0; q0 < nq; q0 += NQ) {
+        const int y0 = (pool ? 2 * oy + (q0 >> 1) : oy) - pad;
+        const int x0 = (pool ? 2 * ox + (q0 & 1) : ox) - pad;
+        float lv[NQ][T::NLEAF];
 #pragma unroll
-      for (int l = 0; l < T::NLEAF; ++l) {
-        float acc[NQ];
+        for (int l = 0; l < T::NLEAF; ++l) {
+          float acc[NQ];
 #pragma unroll
-        for (int q = 0; q < NQ; ++q) acc[q] = 0.0f;
-        for (int k = 0; k < K; ++k) {
-          const int e = (n * T::NLEAF + l) * K + k;
-          const int c = min(max(cm[e], 0), C - 1);
-          const int iy = y0 + min(max(ch[e], 0), kernel - 1);
-          const int ix = x0 + min(max(cw[e], 0), kernel - 1);
-          const float wk = w ? w[e] : 1.0f;
-          const int base = (c * H + iy) * W + ix;
-          float xv[NQ];
+          for (int q = 0; q < NQ; ++q) acc[q] = 0.0f;
+          for (int k = 0; k < K; ++k) {
+            const int e = (n * T::NLEAF + l) * K + k;
+            const int c = min(max(cm[e], 0), C - 1);
+            const int iy = y0 + min(max(ch[e], 0), kernel - 1);
+            const int ix = x0 + min(max(cw[e], 0), kernel - 1);
+            const float wk = w ? w[e] : 1.0f;
+            const int base = (c * H + iy) * W + ix;
+            float xv[NQ];
 #pragma unroll
-          for (int q = 0; q < NQ; ++q) {
-            const int dy = q >> 1, dx = q & 1;
-            const bool in = (unsigned)(iy + dy) < (unsigned)H && (unsigned)(ix + dx) < (unsigned)W;
-            const float t = xb[in ? base + dy * W + dx : 0];
-            xv[q] = in ? t : 0.0f;
+            for (int q = 0; q < NQ; ++q) {
+              const int dy = q >> 1, dx = q & 1;
+              const bool in = (unsigned)(iy + dy) < (unsigned)H && (unsigned)(ix + dx) < (unsigned)W;
+              const uint32_t at = xo + (uint32_t)(in ? base + dy * W + dx : 0);
+              const float t = *reinterpret_cast<const float*>(reinterpret_cast<const char*>(xb) +
+                                                              (NARROW ? at * 4u : (uint64_t)at * 4u));
+              xv[q] = in ? t : 0.0f;
+            }
+#pragma unroll
+            for (int q = 0; q < NQ; ++q) acc[q] = fmaf(wk, xv[q], acc[q]);
           }
 #pragma unroll
-          for (int q = 0; q < NQ; ++q) acc[q] = fmaf(wk, xv[q], acc[q]);
+          for (int q = 0; q < NQ; ++q) lv[q][l] = acc[q];
         }
 #pragma unroll
-        for (int q = 0; q < NQ; ++q) lv[q][l] = acc[q];
+        for (int q = 0; q < NQ; ++q) {
+          float val[T::NLEAF + T::NN];
+#pragma unroll
+          for (int l = 0; l < T::NLEAF; ++l) val[l] = lv[q][l];
+          gen_eval<NODE, A, D>(val, par);
+          best = fmaxf(best, val[T::NLEAF + T::NN - 1]);
+        }
       }
-#pragma unroll
-      for (int q = 0; q < NQ; ++q) {
-        float val[T::NLEAF + T::NN];
-#pragma unroll
-        for (int l = 0; l < T::NLEAF; ++l) val[l] = lv[q][l];
-        gen_eval<NODE, A, D>(val, par);
-        best = fmaxf(best, val[T::NLEAF + T::NN - 1]);
+      if constexpr (NARROW) {
+        char* o = reinterpret_cast<char*>(out + (b0 * N + n) * HoWo);
+        *reinterpret_cast<float*>(o + 4u * ((uint32_t)db * (uint32_t)(N * HoWo) + (uint32_t)p)) = best;
+      } else {
+        out[((b0 + db) * N + n) * HoWo + p] = best;
       }
     }
-    out[(b * N + n) * HoWo + p] = best;
   }
 }
 
@@ -490,14 +515,29 @@ int conv_generic_fwd(const float* x, int64_t B, int64_t C, int64_t H, int64_t W,
   const int64_t nblk = cdiv(Ho * Wo, 256);
   SLG_REQUIRE(nblk * B < (1LL << 31) && N < 65536 && C * H * W < (1LL << 31), SLG_E_SHAPE,
               "conv_soft (generic): too large");
-  const int64_t total = B * Ho * Wo, nwork = cdiv(total, 256) * N;
+  const int64_t total = B * Ho * Wo, runs = cdiv(total, 256);
+  // Trees of few taps: four channels a workgroup, which finds its positions once
+  // (walsh depth 1, K = 1, 16 -> 16 at 96x96, B = 512, not pooled: 518 -> 368 us
+  // against one; pooled depth 2, K = 4, 64 taps, 3 -> 64 at 32x32: 254 and 264),
+  // where that leaves 16 workgroups a CU; two where it leaves 8 (B = 8: 9.5 us
+  // with one, 7.9 before the channels of a run followed each other).
+  const int64_t taps = (pool ? 4 : 1) * (int64_t)conv_generic_leaves(node, depth, arity) * K;
+  const int64_t per_cu = runs * N / device_cus();
+  const int cpw = taps > 32 || per_cu < 16 ? 1 : per_cu < 64 ? 2 : 4;
+  const int64_t groups = cdiv(N, cpw), nwork = runs * groups;
+  const int64_t samples = 255 / (Ho * Wo) + 2;  // that a workgroup's 256 positions reach
+  const bool narrow = nwork < (1LL << 24) && total < (1LL << 30) && Ho * Wo < (1LL << 24) - 256 &&
+                      samples * C * H * W < (1LL << 30) && samples * N * Ho * Wo < (1LL << 30);
   return gen_dispatch(node, A, depth, [&](auto nd, auto a_, auto d_) -> int {
     constexpr int NODE = decltype(nd)::value, AA = decltype(a_)::value, DD = decltype(d_)::value;
     auto run = [&](auto nq) -> int {
-      hipLaunchKernelGGL((conv_generic_fwd_kernel<NODE, AA, DD, decltype(nq)::value>),
-                         dim3((unsigned)std::min<int64_t>((nwork + 7) & ~int64_t(7), 1 << 22)),
-                         dim3(256), 0, st, x, (int)C, (int)H, (int)W, (int)N, K, kernel, pad,
-                         (int)pool, (int)Ho, (int)Wo, total, nwork, np, w, cm, ch, cw, out);
+      constexpr int NQ = decltype(nq)::value;
+      auto kern = narrow ? conv_generic_fwd_kernel<NODE, AA, DD, NQ, true>
+                         : conv_generic_fwd_kernel<NODE, AA, DD, NQ, false>;
+      hipLaunchKernelGGL(kern, dim3((unsigned)std::min<int64_t>((nwork + 7) & ~int64_t(7), 1 << 22)),
+                         dim3(256), 0, st, x, (int)C, (int)H, (int)W, (int)N, K, kernel, pad, (int)pool,
+                         (int)Ho, (int)Wo, 1.0f / (float)(Ho * Wo), 1.0f / (float)Wo, total, nwork, (int)groups,
+                         1.0f / (float)groups, cpw, np, w, cm, ch, cw, out);
       SLG_LAUNCH_CHECK("conv_soft (generic)");
       return 0;
     };
