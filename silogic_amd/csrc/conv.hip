@@ -44,8 +44,6 @@ namespace slg {
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-__device__ inline float sigmoidc(float z) { return 1.0f / (1.0f + expf(-z)); }
-
 constexpr int kMaxK = 8;
 constexpr int kQuadThreadsC = 1024;  // quad-layout workgroups (kQuadThreads)
 
@@ -1109,7 +1107,7 @@ __global__ void conv_soft_prep_kernel(const float* __restrict__ conn, int N, int
     }
   } else {
     const int P = 1 << arity;
-    for (int q = 0; q < P; ++q) np[(int64_t)n * P + q] = sigmoidc(raw[(int64_t)n * P + q]);
+    for (int q = 0; q < P; ++q) np[(int64_t)n * P + q] = sigmoid_exact(raw[(int64_t)n * P + q]);
   }
 }
 
@@ -1187,14 +1185,14 @@ __global__ void conv_soft_records_kernel(const float* __restrict__ conn, const i
     }
   } else if (node == SLG_NODE_HYBRID) {
     const int P = 1 << arity, q = slot - LK * (NW + 1);
-    if (q < P) v = sigmoidc(raw[(int64_t)n * P + q]);
+    if (q < P) v = sigmoid_exact(raw[(int64_t)n * P + q]);
   } else {
     // the kept form of conv_tree.h: per group of corners, its polynomial's
     // coefficients (lut_group_coeffs over the group's corner values: the
     // sigmoid of the logits, or the values as given)
     const int P = 1 << arity, q = slot - LK * (NW + 1);
     const float* s_ = raw + (int64_t)n * P;
-    auto val = [&](int i) { return ARR ? s_[i] : sigmoidc(s_[i]); };
+    auto val = [&](int i) { return ARR ? s_[i] : sigmoid_exact(s_[i]); };
     if (q < P) {
       if (arity >= 3) {
         float c[8];

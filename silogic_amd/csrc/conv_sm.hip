@@ -22,12 +22,12 @@
 // -> here): gate16 depth 2, 64 -> 128 channels at 14 x 14, B = 1024: 950 -> 260
 // us (grad 81, gx 126, images 32); LUT6, 128 -> 256 at 16 x 16, B = 512: 2900
 // -> 580 us (route 106, grad 197, gx 219, images 39); walsh depth 2, 64 -> 128
-// at 14 x 14, B = 256: 1470 -> 130 us. What bounds them now: sm_grad and
-// sm_route the vector ALU (LUT6: about 900 instructions per 64 outputs, 190 us
-// at full issue) and LDS; sm_gx the latency of the leaf gradients (each is
-// read by its tree's two channels, and once more by neighbouring strips, from
-// beyond L2: about 350 and 670 MB) at 8-12 waves a CU, which its strips' LDS
-// and registers allow; sm_images the copy rate.
+// at 14 x 14, B = 256: 1470 -> 130 us. What bounds them now (counters of config 3
+// and 5 training steps): sm_grad and sm_route the vector ALU (LUT6: 590 and 440
+// instructions per 64 outputs, 219 us at full issue of the 288) and LDS; sm_gx
+// the latency of the leaf gradients, which it reads 1.6 (gate16: 163 MB from
+// HBM) and 2.8 times (LUT6: 571 MB), each being read by its tree's two channels
+// and by neighbouring strips; sm_images the copy rate.
 //
 // Launches, per round of samples (kSmRoundFloats):
 //   sm_images    x and gy to sample-minor chunks of 64 samples;

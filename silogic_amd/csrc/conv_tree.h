@@ -103,8 +103,6 @@ __device__ inline float conv_tree_eval(const float (&v)[NLEAF], const float* par
   }
 }
 
-__device__ inline float tree_sigmoid(float z) { return 1.0f / (1.0f + expf(-z)); }
-
 // Value of one node with children c[0..A) and parameters p, as the forward
 // through the caches evaluates it.
 template <int NODE, int A>
@@ -114,7 +112,7 @@ __device__ inline float gen_node(const float* c, const float* __restrict__ p) {
     // contraction moves the window position of near-ties
     const float a = c[0], b = c[1];
     const float z = fmaf(p[3], a * b, fmaf(p[2], b, fmaf(p[1], a, p[0])));
-    if constexpr (NODE == SLG_NODE_WALSH) return tree_sigmoid(z);
+    if constexpr (NODE == SLG_NODE_WALSH) return sigmoid_exact(z);
     return z;
   } else if constexpr (NODE == SLG_NODE_HYBRID) {
     int addr = 0;

@@ -1143,7 +1143,7 @@ __device__ inline float4 node_param(int node, const float* raw, int o) {
     const float t0 = r[0], t1 = r[1], t2 = r[2], t3 = r[3];
     return make_float4(((t0 - t1) - t2) + t3, 2.0f * (t1 - t3), 2.0f * (t2 - t3), 4.0f * t3);
   }
-  return make_float4(sigmoidf_(r[0]), sigmoidf_(r[1]), sigmoidf_(r[2]), sigmoidf_(r[3]));
+  return make_float4(sigmoid_exact(r[0]), sigmoid_exact(r[1]), sigmoid_exact(r[2]), sigmoid_exact(r[3]));
 }
 
 __global__ void fc_soft_prep_kernel(const float* __restrict__ conn, int OUT, int K, int node,

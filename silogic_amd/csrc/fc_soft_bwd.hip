@@ -149,7 +149,7 @@ fc_soft_bwd_w_kernel(const float* __restrict__ x, int B, int IN, int OUT, int Kr
   const int t_end = min(n_tiles, (r_b + 1) * tiles_per_range);
   // AHEAD: the next tile's rows (up to NPF quads of inputs per thread) ride in
   // registers while this tile computes: staged between two barriers with
-  // nothing else in flight, three quarters of the wave cycles waited (10000 ->
+  // nothing else in flight, the workgroup waits for every tile (10000 ->
   // 10000, K = 8, B = 4096: 386 -> 318 us; a workgroup with one tile has
   // nothing to overlap, 12.0 against 13.7 us at 2000 -> 2000, B = 256).
   constexpr int NPF = AHEAD ? kBwdAheadQuads : 0;

@@ -30,7 +30,6 @@ __device__ inline void fma_acc(VT& acc, float w, VT v) {
 }
 template <typename T> __device__ inline T zero_vec() { return (T)0.0f; }
 
-__device__ inline float sigmoidf_(float z) { return 1.0f / (1.0f + expf(-z)); }
 // The per-(sample, output) sigmoid of the walsh node: 1 / (1 + 2^(-z log2 e))
 // with the hardware exp2 and reciprocal (v_exp_f32, v_rcp_f32: about 1 ulp
 // each, against some twenty instructions for expf and an IEEE divide). Large

@@ -4,10 +4,10 @@
 // each. As torch operators they were 5-10 launches forward and as many
 // backward per layer (softmax, gate softmax, basis product, sigmoid, stacks
 // and concatenations of tree levels), 3-5 us each on tables of a few hundred
-// KB; a walsh tree block alone took about 90. Forward and backward together,
-// measured before and after: walsh block 64 -> 128 channels, B = 256: 722 ->
-// 326 us; gate16 block: 408 -> 312 us; four 2000-output FC layers, B = 256:
-// 1176 -> 854 us. Each launch takes 3.6-6.4 us at these sizes.
+// KB; a walsh tree block alone took about 90. Each launch here takes 3.6-6.8 us
+// at these sizes. Training steps are bound by the host there: four 2000-output
+// FC layers with cross-entropy, B = 256: 1151 -> 865 us together with the FC
+// kernels' changes.
 //   gate16      c = softmax(logits) @ BASIS                (nodes.py:82-84)
 //   walsh       (a, b)-space coefficients of z, times scale (nodes.py:138-143)
 //   LUT nodes   s = sigmoid(logits)                        (nodes.py:174-178)
@@ -93,8 +93,6 @@ __device__ inline void lp_gate_probs(const float* __restrict__ g, float (&p)[16]
   for (int i = 0; i < 16; ++i) p[i] = p[i] / sum;
 }
 
-__device__ inline float lp_sigmoid(float z) { return 1.0f / (1.0f + expf(-z)); }
-
 __global__ void __launch_bounds__(256) layer_params_kernel(LpArgs a, const float* __restrict__ conn,
                                                            float* __restrict__ w,
                                                            float* __restrict__ np,
@@ -125,7 +123,7 @@ __global__ void __launch_bounds__(256) layer_params_kernel(LpArgs a, const float
   if (!lp_node(a, lut ? t / a.P : t, lv, rr, kr)) return;
   if (lut) {  // a thread per value
     const int e = (int)(t % a.P);
-    np[kr * a.P + e] = lp_sigmoid(a.raw[lv][rr * a.P + e]);
+    np[kr * a.P + e] = sigmoid_exact(a.raw[lv][rr * a.P + e]);
     return;
   }
   float c[4] = {0.0f, 0.0f, 0.0f, 0.0f};

@@ -3,6 +3,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <math.h>
 #include <stdint.h>
 #include <stdio.h>
 #include <string>
@@ -68,6 +69,9 @@ __device__ inline __amdgpu_buffer_rsrc_t uniform_rsrc(const void* p, int bytes) 
   return __builtin_amdgcn_make_buffer_rsrc((void*)(((uint64_t)hi << 32) | (uint64_t)lo), (short)0,
                                            n, kBufferWord3);
 }
+
+// One form for forward and backward: the pooled routing compares its values.
+__device__ inline float sigmoid_exact(float z) { return 1.0f / (1.0f + expf(-z)); }
 
 // q = e / d for 0 <= e < 2^24 and 0 < d < 2^24, with inv = 1.0f / d: the
 // float quotient is within one of the true one, and the remainder test

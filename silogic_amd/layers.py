@@ -340,7 +340,8 @@ class ConvLogicTree(nn.Module):
     of arity 2-6 with at most 36 leaves), stride 1 with ``padding = kernel //
     2``. Gate16 trees of depth 1-4 and depth-1 LUTs run on the LDS-staged
     kernels (records without gradients); the others on the generic tree
-    kernels, with parameters from differentiable torch ops."""
+    kernels. With gradients a plain softmax selection runs as one operator on
+    the layer's own parameters, others on differentiable torch ops."""
 
     def __init__(self, in_channels, out_channels, kernel=3, tree_depth=None,
                  stride=1, padding=1, connect="topk", k=4, n_chan=2,
@@ -458,8 +459,9 @@ class ConvLogicTree(nn.Module):
     @property
     def generic(self):
         """True for trees outside the LDS-staged kernels' set (walsh trees,
-        LUT trees deeper than one level, gate16 trees of depth 5): their
-        parameters come from torch ops, the hard path from per-node tables."""
+        LUT trees deeper than one level, gate16 trees of depth 5): without
+        gradients their parameters come from torch ops; the hard path from
+        per-node tables."""
         if self.node_name == "gate16":
             return self.d > 4
         return self.node_name == "walsh" or self.d != 1
