@@ -16,6 +16,8 @@
 // average, one call in twenty by more than 10%, the worst 2.9 times (always along
 // samples: 18% on average, 20 times). Not by whether the input gradient is
 // wanted: the other gradients are the same bits with and without it.
+#include <array>
+
 #include "conv_pos.h"
 #include "conv_sm.h"
 #include "conv_tree.h"
@@ -29,9 +31,9 @@ struct ConvBwdChoice {
 };
 
 // path: SLG_CONV_BWD_AUTO or the kernels to take, where they take the sizes.
-static ConvBwdChoice conv_bwd_choose(int path, int64_t B, int64_t C, int64_t H, int64_t W, int64_t N,
-                                     int node, int depth, int arity, int K, int pad, bool pool,
-                                     bool want_x) {
+static ConvBwdChoice conv_bwd_estimate(int path, int64_t B, int64_t C, int64_t H, int64_t W, int64_t N,
+                                       int node, int depth, int arity, int K, int pad, bool pool,
+                                       bool want_x) {
   ConvBwdChoice c{};
   c.raw = pool && (node == SLG_NODE_GATE16 || node == SLG_NODE_MULTILINEAR2) &&
           !conv_forward_on_lds(C, H, W, N, node, depth, arity, K, pad, pool);
@@ -64,6 +66,29 @@ static ConvBwdChoice conv_bwd_choose(int path, int64_t B, int64_t C, int64_t H, 
   }
   c.floats = workspace(c.path, want_x, nullptr);
   return c;
+}
+
+// The last few choices of a thread, by everything they depend on: the workspace
+// query and the call that follows it ask the same, each step again (2-3 us each).
+static ConvBwdChoice conv_bwd_choose(int path, int64_t B, int64_t C, int64_t H, int64_t W, int64_t N,
+                                     int node, int depth, int arity, int K, int pad, bool pool,
+                                     bool want_x) {
+  using Key = std::array<int64_t, 15>;
+  struct Kept {
+    Key key;
+    ConvBwdChoice choice;
+  };
+  constexpr int kKept = 16;
+  static thread_local Kept kept[kKept];  // all zero: no choice has zero channels
+  static thread_local unsigned next = 0;
+  const Key key{path, B, C, H, W, N, node, depth, arity, K, pad, pool, want_x, device_cus(),
+                device_lds_bytes()};
+  for (const Kept& k : kept)
+    if (k.key == key) return k.choice;
+  Kept& k = kept[next++ % kKept];
+  k.choice = conv_bwd_estimate(path, B, C, H, W, N, node, depth, arity, K, pad, pool, want_x);
+  k.key = key;
+  return k.choice;
 }
 
 }  // namespace slg

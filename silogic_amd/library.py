@@ -226,45 +226,45 @@ def _gradients(x, *wanted):
 
 @torch.library.custom_op(f"{_NS}::fc_layer", mutates_args=())
 def fc_layer(x: Tensor, cand: Tensor, conn: Optional[Tensor], raw: Tensor, node_kind: int,
-             inv_tau: float) -> Tuple[Tensor, Tensor, Tensor, Tensor]:
+             inv_tau: float) -> Tuple[Tensor, Tensor, Tensor]:
     """Gate layer: ``x [B,IN]``, ``cand/conn [OUT,A,K]``, ``raw`` the node's
-    parameters -> ``(y [B,OUT], w [OUT,A,K], npar, probs)``. ``A = 2`` gate16
-    and walsh nodes, and arity-2 multilinear ones, as ``fc_soft``; ``probs``
-    ``[OUT,1,16]`` (gate16) or empty."""
+    parameters -> ``(y [B,OUT], w [OUT,A,K], kept)``. ``A = 2`` gate16
+    and walsh nodes, and arity-2 multilinear ones, as ``fc_soft``; ``kept`` as
+    :func:`ops.layer_params` returns it."""
     ops.require_gpu(x, cand, conn, raw)
     if tuple(raw.shape) != (cand.shape[0], 16 if node_kind == ops.GATE16 else 4):
         raise ValueError(f"fc_layer: parameters {tuple(raw.shape)} for {cand.shape[0]} outputs")
     cand = ops._c(cand, torch.int32)
-    w, npar, probs = ops.layer_params(conn, tuple(cand.shape), [raw], node_kind, 2)
-    npar = npar.view(-1, 4)
-    return ops._fc_soft_launch(ops._as_f32(x), cand, w, npar, node_kind, inv_tau), w, npar, probs
+    w, kept = ops.layer_params(conn, tuple(cand.shape), [raw], node_kind, 2)
+    npar = kept[:cand.shape[0]] if node_kind == ops.GATE16 else kept
+    return ops._fc_soft_launch(ops._as_f32(x), cand, w, npar, node_kind, inv_tau), w, kept
 
 
 @fc_layer.register_fake
 def _(x, cand, conn, raw, node_kind, inv_tau):
     OUT = cand.shape[0]
-    return _layer_outputs(x, (x.shape[0], OUT), cand.shape, (OUT, 4),
-                          (OUT, 1, 16) if node_kind == ops.GATE16 else (0,))
+    return _layer_outputs(x, (x.shape[0], OUT), cand.shape,
+                          (OUT * (5 if node_kind == ops.GATE16 else 1), 4))
 
 
 @torch.library.custom_op(f"{_NS}::fc_layer_bwd", mutates_args=())
-def fc_layer_bwd(x: Tensor, cand: Tensor, w: Tensor, npar: Tensor, probs: Tensor, node_kind: int,
-                 inv_tau: float, gy: Tensor, need_x: bool, need_conn: bool,
+def fc_layer_bwd(x: Tensor, cand: Tensor, w: Tensor, kept: Tensor, node_kind: int, inv_tau: float,
+                 gy: Tensor, need_x: bool, need_conn: bool,
                  need_raw: bool) -> Tuple[Tensor, Tensor, Tensor]:
     """``(gx, gconn, graw)`` of fc_layer; unneeded ones are empty."""
-    got = ops.fc_soft_bwd(x, cand, w, npar, node_kind, inv_tau, gy, need_x, need_conn, need_raw)
+    got = ops.fc_soft_bwd(x, cand, w, kept, node_kind, inv_tau, gy, need_x, need_conn, need_raw)
     if got is None:
         raise NotImplementedError("fc_layer backward: shape outside the HIP kernels "
                                   "(K > 16 or 2*OUT*K >= 2^31)")
     gx, gw, gn = got
-    gconn, (graw,) = ops.layer_params_bwd(w, gw, probs if node_kind == ops.GATE16 else npar, [1],
-                                          node_kind, 2, 1.0, gn, need_conn, [need_raw])
+    gconn, (graw,) = ops.layer_params_bwd(w, gw, kept, [1], node_kind, 2, 1.0, gn, need_conn, [need_raw],
+                                          4 * w.shape[0] if node_kind == ops.GATE16 else 0)
     return tuple(g if g is not None else _empty(x)
                  for g in (gx, gconn, None if graw is None else graw.squeeze(1)))
 
 
 @fc_layer_bwd.register_fake
-def _(x, cand, w, npar, probs, node_kind, inv_tau, gy, need_x, need_conn, need_raw):
+def _(x, cand, w, kept, node_kind, inv_tau, gy, need_x, need_conn, need_raw):
     raw = (cand.shape[0], 16 if node_kind == ops.GATE16 else 4)
     return _gradients(x, (x.shape, need_x), (w.shape, need_conn), (raw, need_raw))
 
@@ -298,8 +298,7 @@ def fc_lut_layer(x: Tensor, cand: Tensor, conn: Optional[Tensor], logits: Tensor
         raise ValueError(f"fc_lut_layer: logits {tuple(logits.shape)} for candidates "
                          f"{tuple(cand.shape)}")
     cand = ops._c(cand, torch.int32)
-    w, s, _ = ops.layer_params(conn, tuple(cand.shape), [logits], ops.HYBRID, cand.shape[1])
-    s = s.view(logits.shape)
+    w, s = ops.layer_params(conn, tuple(cand.shape), [logits], ops.HYBRID, cand.shape[1])
     return ops._fc_lut_launch(ops._as_f32(x), cand, w, s, hybrid), w, s
 
 
@@ -497,8 +496,10 @@ def conv_layer(x: Tensor, conn: Optional[Tensor], l0: Tensor, l1: Optional[Tenso
         # autocast runs the product in 16 bits, a default dtype makes the ones
         w, npar, probs = (ops._c(t, torch.float32) for t in (w, npar, probs))
     else:
-        w, npar, probs = ops.layer_params(conn, tuple(cm.shape), levels, node_kind,
-                                          2 if node_kind == ops.WALSH else arity, scale)
+        w, npar = ops.layer_params(conn, tuple(cm.shape), levels, node_kind,
+                                   2 if node_kind == ops.WALSH else arity, scale)
+        npar, probs = npar.view(cm.shape[0], -1, ops.tree_shape(node_kind, depth, arity)[2]), \
+            x.new_empty((0,), dtype=torch.float32)
     y = ops._conv_soft_launch(ops._as_f32(x), npar, w, cm, ch, cw, node_kind, depth, arity, K, pad,
                               pool)
     return y, w, npar, probs

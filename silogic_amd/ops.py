@@ -217,10 +217,10 @@ def _levels_f32(levels):
 
 
 def layer_params(conn, w_shape, levels, kind, arity, scale=1.0):
-    """``(w, npar, probs)`` of a layer from its parameters in one launch: ``w``
-    (shape ``[N, ..., K]``) = softmax of ``conn`` (ones for None), ``npar``
-    ``[N, nodes, P]`` from the raw parameters of every tree level, ``probs``
-    gate16's softmax ``[N, nodes, 16]`` (other nodes: empty)."""
+    """``(w, kept)`` of a layer from its parameters in one launch: ``w``
+    (shape ``[N, ..., K]``) = softmax of ``conn`` (ones for None), ``kept`` the
+    node parameters from the raw ones of every tree level, a row of P each
+    (``N * nodes``), for gate16 followed by its softmax, 16 each, as rows too."""
     if conn is not None and tuple(conn.shape) != tuple(w_shape):
         raise ValueError(f"layer_params: conn {tuple(conn.shape)} for candidates {tuple(w_shape)}")
     N, K = w_shape[0], w_shape[-1]
@@ -229,31 +229,32 @@ def layer_params(conn, w_shape, levels, kind, arity, scale=1.0):
     nodes, NN = _level_args(levels, N, 16 if kind == GATE16 else P)
     dev = levels[0].device
     w = torch.empty(w_shape, device=dev, dtype=torch.float32)
-    npar = torch.empty((N, NN, P), device=dev, dtype=torch.float32)
-    probs = torch.empty((N, NN, 16) if kind == GATE16 else 0, device=dev, dtype=torch.float32)
+    kept = torch.empty((N * NN * (5 if kind == GATE16 else 1), P), device=dev, dtype=torch.float32)
+    npar = kept.data_ptr()
     _lib.call("slg_layer_params", _p(conn), w.numel() // K, K, len(levels), _ptrs(levels), nodes, N,
-              kind, arity, float(scale), _p(w), _p(npar), _p(probs) if kind == GATE16 else None,
-              _stream(levels[0]))
-    return w, npar, probs
+              kind, arity, float(scale), _p(w), ctypes.c_void_p(npar),
+              ctypes.c_void_p(npar + 4 * N * NN * P) if kind == GATE16 else None, _stream(levels[0]))
+    return w, kept
 
 
-def layer_params_bwd(w, gw, kept, nodes, kind, arity, scale, gnp, need_conn, need_levels):
+def layer_params_bwd(w, gw, kept, nodes, kind, arity, scale, gnp, need_conn, need_levels, skip=0):
     """``(gconn, [level gradients [N, m, P]])`` from the gradients of ``w`` and
-    ``npar`` (None where not needed) and what :func:`layer_params` returned,
-    ``kept`` (``probs`` for gate16, ``npar`` for LUTs, unused for walsh):
-    nothing is read from the parameters again, which may have changed since.
-    ``nodes``: nodes per channel of each level."""
+    the node parameters (None where not needed) and what the forward derived,
+    ``kept`` past its first ``skip`` values (gate16: the probabilities, LUTs: the
+    node parameters, walsh: unused): nothing is read from the parameters again,
+    which may have changed since. ``nodes``: nodes per channel of each level."""
     N, K = w.shape[0], w.shape[-1]
     P = 16 if kind == GATE16 else 4 if kind == WALSH else 2 ** arity
     w, kept = _c(w, torch.float32), _quads(_c(kept, torch.float32))
-    if kind != WALSH and kept.numel() != N * sum(nodes) * P:
+    if kind != WALSH and kept.numel() - skip != N * sum(nodes) * P:
         raise ValueError(f"layer_params_bwd: kept {tuple(kept.shape)} for {N} x {nodes} nodes")
     gconn = torch.empty_like(w) if need_conn else None
     graw = [torch.empty((N, m, P), device=w.device, dtype=torch.float32) if n else None
             for m, n in zip(nodes, need_levels)]
     _lib.call("slg_layer_params_bwd", _p(w), _p(gw), w.numel() // K, K, len(nodes),
               (ctypes.c_int32 * len(nodes))(*nodes), N, kind, arity, float(scale),
-              None if kind == WALSH else _p(kept), _p(gnp), _p(gconn), _ptrs(graw), _stream(w))
+              None if kind == WALSH else ctypes.c_void_p(kept.data_ptr() + 4 * skip), _p(gnp),
+              _p(gconn), _ptrs(graw), _stream(w))
     return gconn, graw
 
 
