@@ -22,5 +22,5 @@ def test_a_backward_without_kernels_says_so(monkeypatch):
     monkeypatch.setattr(ops, "fc_soft_bwd", lambda *a: None)
     t = torch.zeros
     with pytest.raises(NotImplementedError, match="fc_layer backward"):
-        library.fc_layer_bwd(t(1, 3), t(2, 2, 1, dtype=torch.int32), t(2, 2, 1), t(2, 4), t(2, 1, 16),
-                             ops.GATE16, 1.0, t(1, 2), True, True, True)
+        library.fc_layer_bwd(t(1, 3), t(2, 2, 1, dtype=torch.int32), t(2, 2, 1), t(10, 4), ops.GATE16, 1.0,
+                             t(1, 2), True, True, True)
