@@ -12,9 +12,9 @@
 // it would launch, and the shortest is taken. The factors were fitted to 4700
 // random shapes (1-1024 samples, 1-512 channels, maps of 4-128, kernels 1-7,
 // every node kind, pooled and not, each timed on all three): the estimates
-// scatter by 25-30%; the choice is 1.8% slower than the best of the three on
-// average, one call in twenty by more than 10%, the worst 2.9 times (always along
-// samples: 18% on average, 20 times). Not by whether the input gradient is
+// scatter by 25-30%; the choice is 1.9% slower than the best of the three on
+// average, by more than 10% for 6% of them, the worst 3.5 times (always along
+// samples: 17% on average, 20 times). Not by whether the input gradient is
 // wanted: the other gradients are the same bits with and without it.
 #include <array>
 
