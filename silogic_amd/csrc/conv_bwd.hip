@@ -5,10 +5,10 @@
 //
 // Lanes along samples do the least work, but in units of 64 samples, and few
 // samples leave serial chains (an output row of a tree, the taps of a channel)
-// that the chip waits for. 16 -> 32 channels, 5 x 5, 96 x 96, 2 pooled samples,
+// that the chip waits for. 16 -> 32 channels, 5 x 5, 96 x 96, one pooled sample,
 // along samples / positions / generic: gate16 depth 2, K = 4: 759 / 352 / 113
 // us; 16 of them: 676 / 389 / 547; 64 -> 128, 3 x 3, 14 x 14, 256 samples: 114 /
-// 297 / 580. No one size divides them, so each file estimates its time from what
+// 297 / 1417. No one size divides them, so each file estimates its time from what
 // it would launch, and the shortest is taken. The factors were fitted to 4700
 // random shapes (1-1024 samples, 1-512 channels, maps of 4-128, kernels 1-7,
 // every node kind, pooled and not, each timed on all three): the estimates
